@@ -26,14 +26,23 @@ namespace ugbsa {
 // is unrolled by 2).  Half blocks keep the live set at about 470 registers:
 // O^T 128, two S 64, P 16, Q 64 (in AGPRs, read there by the MFMAs), two K
 // 64, two V^T 64.
-// With SB (head_dim 256) K / V^T keep one set each: K(u+2) requested after
-// phase 1 and V^T(u+1) after phase 2, each a phase ahead of use; phase 1
-// forms the second half of P(u) beside the S(u+1) MFMAs, and phase 2 forms
-// the lane maxima of S(u+1), tests them against the lazy threshold and then
-// forms the first half of P(u+1) (the rescale follows phase 2 when an offset
-// moved).  Head_dim 256 (QLDS) doubles O^T, K and V^T, so Q moves to LDS and
-// O^T (256 registers for 64 rows) to the AGPR file (OA), where only the P.V
-// MFMAs touch it.
+// With SB (head_dim 64 and 256) K / V^T keep one set each: K(u+2) requested
+// after phase 1 and V^T(u+1) after phase 2, each a phase ahead of use.
+// Head_dim 256 (QLDS, OA) doubles O^T, K and V^T, so Q moves to LDS and
+// O^T (256 registers for 64 rows) to the AGPR file, where only the P.V
+// MFMAs touch it; phase 1 forms the second half of P(u) beside the S(u+1)
+// MFMAs, and phase 2 forms the lane maxima of S(u+1), tests them against the
+// lazy threshold and then forms the first half of P(u+1) (the rescale
+// follows phase 2 when an offset moved).
+// Head_dim 64 halves them instead: with one K / V^T set and Q in LDS the live
+// set is 244 registers, so two wavefronts share a SIMD.  It is bound by the
+// softmax's VALU work (the 32 exponentials, FMAs, adds and 16 packs of a half
+// block take ~830 issue cycles beside 512 cycles of MFMAs), which the second
+// wavefront keeps issuing while the first waits.  It keeps the row-sum test
+// (commit), 28 VALU instructions per half block fewer than testing the lane
+// maxima.  Attention of 2 x 16 heads x 8192 tokens, us per call with 32 / 128
+// listed blocks: one wavefront per SIMD 212 / 360, two with the lane maxima
+// 199 / 360, two with the row sums 186 / 339 (816 TFLOP/s).
 // The tile's kv_idx row is compacted into LDS once (visited blocks only), so
 // sentinel and invisible slots cost nothing in the loop.
 // Per-wave LDS bytes of attn_fwd_pipe_kernel: Q fragments (QLDS), block
@@ -51,7 +60,7 @@ __host__ __device__ inline int pipe_wave_lds(int D, int NT, bool qlds, int k_slo
 constexpr int kGenBlocks = 512;
 
 template <typename E, int D, int NT, bool QLDS, bool SB, bool OA>
-__global__ __launch_bounds__(64 * (4 / NT)) void attn_fwd_pipe_kernel(
+__global__ __launch_bounds__(64 * (4 / NT), D == 64 ? 2 : 1) void attn_fwd_pipe_kernel(
     const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
     const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
     const uint16_t* __restrict__ vt, const int32_t* __restrict__ kv_idx,
@@ -341,10 +350,10 @@ __global__ __launch_bounds__(64 * (4 / NT)) void attn_fwd_pipe_kernel(
       }
     }
   };
-  // Lazy offsets with SB, tested lane-locally: a row's offset m only moves
+  // Lazy offsets with OA, tested lane-locally: a row's offset m only moves
   // when some lane's max of its raw scores exceeds
   // thr = (m + kLazyLog2) / sl2; the cross-lane row max is only formed inside
-  // the (rare) rescale.  Without SB the row sums are tested instead (commit)
+  // the (rare) rescale.  Without OA the row sums are tested instead (commit)
   // and lane maxima are formed only when that test fires.
   float thr[NT], rm[NT], tm[NT][4];
 #pragma unroll
@@ -431,7 +440,7 @@ __global__ __launch_bounds__(64 * (4 / NT)) void attn_fwd_pipe_kernel(
     if (kk == 7) {
       sum[nt] += p[nt][7];
       w[nt][3] = E::pack2(p[nt][6], p[nt][7]);
-      if constexpr (SB) l[nt] += sum[nt];
+      if constexpr (OA) l[nt] += sum[nt];
       pb[nt] = __builtin_bit_cast(bf16x8, u32x4{w[nt][0], w[nt][1], w[nt][2], w[nt][3]});
     }
   };
@@ -449,13 +458,10 @@ __global__ __launch_bounds__(64 * (4 / NT)) void attn_fwd_pipe_kernel(
   // The two phases of a step are woven by hand (one wave per SIMD issues in
   // order, so VALU work has to sit between the MFMAs of the instruction
   // stream); sched_barrier keeps the compiler from regrouping them.
-  // With SB:
-  //   phase 1: S^T(u+1) (NM1 MFMAs) || softmax of S(u) (all 8 NT elements)
-  //   phase 2: O^T += V^T P^T(u) (NM2 MFMAs) || the row-max test of S(u+1)
-  // Without SB:
-  //   phase 1: S^T(u+1) || softmax elements [4 NT, 8 NT) of S(u)
-  //   phase 2: O^T += V^T P^T(u) || softmax elements [0, 4 NT) of S(u+1)
-  // with the lazy test after phase 1, on the row sums (commit).
+  //   phase 1: S^T(u+1) (NM1 MFMAs) || softmax elements [4 NT, 8 NT) of S(u)
+  //   phase 2: O^T += V^T P^T(u) (NM2 MFMAs) || softmax elements [0, 4 NT) of
+  //            S(u+1), with OA after the row-max test of S(u+1); without OA
+  //            the lazy test runs on the row sums after phase 1 (commit).
   constexpr int NM1 = 2 * NT * KS, P1 = NM1 / 2;
   constexpr int E1ST = 4 * NT;                      // first softmax element of phase 1
   constexpr int NE1 = 8 * NT - E1ST;                // softmax elements of phase 1
@@ -514,7 +520,7 @@ __global__ __launch_bounds__(64 * (4 / NT)) void attn_fwd_pipe_kernel(
       o[dt1][nt1] = E::mfma(vf[dt1], pb[nt1], o[dt1][nt1]);
     }
   };
-  // Phase 2 with SB: O^T += V^T . P^T(u) row set by row set (pairs over the
+  // Phase 2 with OA: O^T += V^T . P^T(u) row set by row set (pairs over the
   // head dims of one row set, then the next), woven with the lazy test of
   // S(u+1) over the first row set's pairs and, once it has passed, the
   // first half of the softmax of S(u+1): row set nt' of P(u+1) is formed
@@ -573,7 +579,7 @@ __global__ __launch_bounds__(64 * (4 / NT)) void attn_fwd_pipe_kernel(
 #pragma unroll
     for (int j = 0; j < P2; ++j) pv_pair(vf, j);
   };
-  // Phase 2 without SB: the P.V MFMAs row set by row set; once
+  // Phase 2 without OA: the P.V MFMAs row set by row set; once
   // row set nt' of P(u) has been read, row set nt' of P(u+1) is computed
   // (elements 8 nt' .. 8 nt' + 7 of S(u+1), over the next DT / 2 pairs).
   // on_pair(j) issues this step's share of the next K loads before pair j,
@@ -597,7 +603,7 @@ __global__ __launch_bounds__(64 * (4 / NT)) void attn_fwd_pipe_kernel(
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  // The lazy test without SB, after the softmax of half block st
+  // The lazy test without OA, after the softmax of half block st
   // is complete: a lane's sum of its eight P values above 2^kLazyLog2 means
   // the offset m of that row is stale (some P exceeded the lazy bound).
   // Then the offsets move to the half block's row maxima, l and O are
@@ -620,15 +626,18 @@ __global__ __launch_bounds__(64 * (4 / NT)) void attn_fwd_pipe_kernel(
 
   SBuf sa, sb;
   if constexpr (SB) {
-    // One K and one V^T set (at head_dim 256 two would take 256 registers).
+    // One K and one V^T set (at head_dim 256 two would take 256 registers, at
+    // head_dim 64 they would cost the second wavefront per SIMD).
     // Step u: S(u) in cur (its first half already softmaxed), K(u+1) in ka,
     // V(u) in va; K(u+2) is requested after phase 1 and V(u+1) after
-    // phase 2 — a phase ahead of use (about 2000 cycles at head_dim 256).
+    // phase 2 — a phase ahead of use (about 2000 cycles at head_dim 256,
+    // about 500 at head_dim 64, where the other wavefront covers the rest).
     auto step1 = [&](SBuf& cur, SBuf& nxt, int u) {
       const int rk = blk_raw(u + 2), rm1 = blk_raw(u + 1);
       asm volatile("" : "+v"(lane_b));
       phase1(cur, nxt, ka);
       load_k(uni(rk), clamp_u(u + 2) & 1, ka);
+      if constexpr (!OA) commit(cur);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         u32x4 pin = __builtin_bit_cast(u32x4, pb[nt]);
@@ -636,10 +645,15 @@ __global__ __launch_bounds__(64 * (4 / NT)) void attn_fwd_pipe_kernel(
         pb[nt] = __builtin_bit_cast(bf16x8, pin);
       }
       mask(nxt, uni(rm1), (u + 1) & 1, mbits(u + 1));
-      float alpha[NT];
-      const bool moved = phase2(nxt, va, alpha);
-      load_v(uni(rm1), (u + 1) & 1, va);
-      if (__builtin_expect(moved, 0)) scale_o(alpha);
+      if constexpr (OA) {
+        float alpha[NT];
+        const bool moved = phase2(nxt, va, alpha);
+        load_v(uni(rm1), (u + 1) & 1, va);
+        if (__builtin_expect(moved, 0)) scale_o(alpha);
+      } else {
+        phase2s(nxt, va, [](int) {}, [](int) {});
+        load_v(uni(rm1), (u + 1) & 1, va);
+      }
     };
     if (nv > 0) {
       const int b0 = uni(blk_raw(0));
@@ -661,6 +675,7 @@ __global__ __launch_bounds__(64 * (4 / NT)) void attn_fwd_pipe_kernel(
       step1(sa, sb, u);
 #pragma unroll
       for (int e = E1ST; e < 8 * NT; ++e) softmax_elem(sb, e);
+      if constexpr (!OA) commit(sb);
       pv(va);
     }
   }
