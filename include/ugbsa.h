@@ -247,6 +247,22 @@ int ugbsa_attn_fwd(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m, int6
                    int64_t so_h, int64_t so_m, int64_t so_d, void* workspace,
                    int64_t workspace_elems, void* stream);
 
+/* fp32 elements of a ugbsa_decode workspace (0: none is needed). */
+int64_t ugbsa_decode_workspace_elems(int B, int H, int Hk, int N, int D);
+
+/* Decode — attention of one query row per head over all N keys of its KV head
+ * (no mask), the dispatcher's Q == 1 branch (src/sparse_attention.py:757-767).
+ * q [B, H, 1, D], k/v [B, Hk, N, D] in dtype, out [B, H, D] in dtype with any
+ * b and h strides; B, H <= 65535.  The keys are split over workgroups whose
+ * partial results go through workspace (at least
+ * ugbsa_decode_workspace_elems fp32; NULL where that is 0). */
+int ugbsa_decode(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m, int64_t sq_d,
+                 const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n, int64_t sk_d,
+                 const void* v, int64_t sv_b, int64_t sv_h, int64_t sv_n, int64_t sv_d, int B,
+                 int H, int Hk, int N, int D, int dtype, float scale, void* out, int64_t so_b,
+                 int64_t so_h, int64_t so_d, float* workspace, int64_t workspace_elems,
+                 void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -61,6 +61,11 @@ SIGNATURES = {
                             _p, _i64, _i64, _i64, _i64,
                             _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _f,
                             _p, _i64, _i64, _i64, _i64, _p, _i64, _p]),
+    "ugbsa_decode_workspace_elems": (_i64, [_i, _i, _i, _i, _i]),
+    "ugbsa_decode": (_i, [_p, _i64, _i64, _i64, _i64,
+                          _p, _i64, _i64, _i64, _i64,
+                          _p, _i64, _i64, _i64, _i64,
+                          _i, _i, _i, _i, _i, _i, _f, _p, _i64, _i64, _i64, _p, _i64, _p]),
 }
 ABI_VERSION = 4
 
@@ -103,7 +108,7 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)   # no Stream object per launch
 
 
 def ptr(t) -> int | None:

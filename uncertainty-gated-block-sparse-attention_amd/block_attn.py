@@ -92,6 +92,57 @@ def block_sparse_attn_v2(q, k, v, kv_idx, scale, block_n=64, block_m=64,
     return out
 
 
+def _unwatched(q, k, v):
+    """Whether a launch on the tensors' data pointers is all there is to a call: dense tensors,
+    outside autograd, autocast, tracing, modes and functional transforms."""
+    wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+    return not ((torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad))
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch.is_autocast_enabled("cuda") or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
+                or wrapped(q) or wrapped(k) or wrapped(v)
+                or q.is_nested or k.is_nested or v.is_nested
+                or not (q.layout is k.layout is v.layout is torch.strided))
+
+
+def decode_attn(q, k, v, scale):
+    """Attention of one query row per head over every key of its KV head (HIP).
+
+    q [B, H, 1, D]; k, v [B, Hk, N, D].  Returns [B, 1, H, D] contiguous, the dispatcher's
+    layout, or None for a call the kernel does not take, which is SDPA's then: anything but
+    bf16 / fp16 tensors of one device, head_dim 64, 128 or 256, in a layout read in place (unit
+    head_dim stride, 16-byte aligned rows), with nothing watching the call.
+    """
+    if not (type(q) is type(k) is type(v) is torch.Tensor and q.is_cuda and k.is_cuda and v.is_cuda
+            and isinstance(scale, float) and q.dim() == 4 and k.dim() == 4
+            and (q.dtype is torch.bfloat16 or q.dtype is torch.float16)
+            and k.dtype is q.dtype and v.dtype is q.dtype and _unwatched(q, k, v)):
+        return None
+    B, H, M, D = q.shape
+    Bk, Hk, N, Dk = k.shape
+    if not (M == 1 and (D == 128 or D == 64 or D == 256) and Bk == B and Dk == D
+            and v.shape == k.shape and 0 < B <= 65535 and 0 < H <= 65535 and Hk > 0
+            and H % Hk == 0 and 0 < N < 1 << 30):
+        return None
+    sq, sk, sv = q.stride(), k.stride(), v.stride()
+    pq, pk, pv = q.data_ptr(), k.data_ptr(), v.data_ptr()
+    device, index = q.device, q.get_device()
+    if not (sq[3] == sk[3] == sv[3] == 1 and (pq | pk | pv) & 15 == 0
+            and (sq[0] | sq[1] | sq[2] | sk[0] | sk[1] | sk[2] | sv[0] | sv[1] | sv[2]) & 7 == 0
+            and k.get_device() == index and v.get_device() == index
+            and torch._C._cuda_getDevice() == index):
+        return None
+    lib = _capi.lib()
+    out = torch.empty((B, 1, H, D), dtype=q.dtype, device=device)
+    n = lib.ugbsa_decode_workspace_elems(B, H, Hk, N, D) if N >= 512 else 0   # one split below
+    ws = torch.empty(n, dtype=torch.float32, device=device) if n else None
+    _capi.check(lib.ugbsa_decode(
+        pq, *sq, pk, *sk, pv, *sv, B, H, Hk, N, D, _capi.dtype_code(q.dtype), scale,
+        out.data_ptr(), H * D, D, 1, None if ws is None else ws.data_ptr(), n,
+        _capi.stream_ptr(device)), "decode")
+    return out
+
+
 def keep_kv_idx(keep, block_m=64, want_rowmask=True):
     """HIP compaction of a device keep mask [B, H, M, NB] (bool).
 

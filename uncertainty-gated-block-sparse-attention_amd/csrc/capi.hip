@@ -460,4 +460,36 @@ int ugbsa_router_rows(const float* margin, int B, int H, int M, int NB, int grai
                     "router_rows");
 }
 
+int64_t ugbsa_decode_workspace_elems(int B, int H, int Hk, int N, int D) {
+  if (check_dims(B, H, Hk, D, UGBSA_DTYPE_BF16) || N < 1) return 0;
+  const int64_t splits = ugbsa::decode_splits(B, H, Hk, N, D);
+  return splits == 1 ? 0 : static_cast<int64_t>(B) * H * splits * (D + 2);
+}
+
+int ugbsa_decode(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m, int64_t sq_d,
+                 const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n, int64_t sk_d,
+                 const void* v, int64_t sv_b, int64_t sv_h, int64_t sv_n, int64_t sv_d, int B,
+                 int H, int Hk, int N, int D, int dtype, float scale, void* out, int64_t so_b,
+                 int64_t so_h, int64_t so_d, float* workspace, int64_t workspace_elems,
+                 void* stream) {
+  int rc = check_dims(B, H, Hk, D, dtype);
+  if (rc) return rc;
+  if ((rc = check_bf16_operand("q", q, sq_b, sq_h, sq_m, sq_d))) return rc;
+  if ((rc = check_bf16_operand("k", k, sk_b, sk_h, sk_n, sk_d))) return rc;
+  if ((rc = check_bf16_operand("v", v, sv_b, sv_h, sv_n, sv_d))) return rc;
+  if (N < 1) return fail(UGBSA_EARG, "N must be positive");
+  if (B > 65535 || H > 65535) return fail(UGBSA_EARG, "B and H must be at most 65535 (B=%d, H=%d)", B, H);
+  if (out == nullptr || so_d != 1) return fail(UGBSA_ELAYOUT, "out must be non-null with unit head_dim stride");
+  const int64_t need = ugbsa_decode_workspace_elems(B, H, Hk, N, D);
+  if (need > 0 && (workspace == nullptr || workspace_elems < need))
+    return fail(UGBSA_EARG, "workspace of %lld floats is smaller than ugbsa_decode_workspace_elems (%lld)",
+                (long long)workspace_elems, (long long)need);
+  return hip_result(ugbsa::launch_decode(static_cast<const uint16_t*>(q), sq_b, sq_h,
+                                         static_cast<const uint16_t*>(k), sk_b, sk_h, sk_n,
+                                         static_cast<const uint16_t*>(v), sv_b, sv_h, sv_n, B, H,
+                                         Hk, N, D, dtype, scale, static_cast<uint16_t*>(out), so_b,
+                                         so_h, workspace, static_cast<hipStream_t>(stream)),
+                    "decode");
+}
+
 }  // extern "C"

@@ -136,4 +136,13 @@ hipError_t launch_keep_kv_idx(const uint8_t* keep, int B, int H, int M, int NB, 
                               int32_t* kv_idx, uint64_t* rowmask, int32_t* counts,
                               hipStream_t stream);
 
+// Decode attention (decode.hip): q [B, H, 1, D] over k / v [B, Hk, N, D] into
+// out, ws holding B * H * decode_splits() * (D + 2) fp32 when that is above 1.
+int decode_splits(int B, int H, int Hk, int N, int D);
+hipError_t launch_decode(const uint16_t* q, int64_t sq_b, int64_t sq_h, const uint16_t* k,
+                         int64_t sk_b, int64_t sk_h, int64_t sk_n, const uint16_t* v, int64_t sv_b,
+                         int64_t sv_h, int64_t sv_n, int B, int H, int Hk, int N, int D, int elem,
+                         float scale, uint16_t* out, int64_t so_b, int64_t so_h, float* ws,
+                         hipStream_t stream);
+
 }  // namespace ugbsa

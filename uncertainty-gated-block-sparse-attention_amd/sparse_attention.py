@@ -50,7 +50,7 @@ import torch
 import torch.nn.functional as F
 
 import _capi
-from block_attn import attn_workspace, block_sparse_attn, block_sparse_attn_v2
+from block_attn import attn_workspace, block_sparse_attn, block_sparse_attn_v2, decode_attn
 
 BLOCK = 64   # tokens per selection block (src/sparse_attention.py:51)
 
@@ -471,7 +471,10 @@ def block_sparse_attention(module, query, key, value, attention_mask,
     """HF attention function (src/sparse_attention.py:751-806).
 
     query [B, H, S, D]; key / value [B, Hk, S, D] as transformers passes them
-    (before repeat_kv).  Dense SDPA for ``mode == "dense"`` or decode (Q == 1);
+    (before repeat_kv).  Decode (Q == 1) attends to every key: the HIP decode
+    kernel where ``decode_attn`` takes the call (the library's flash kernel
+    runs one workgroup per query head: 1151 us against 19 at 28/4 heads and 32K
+    keys), else dense SDPA, as for ``mode == "dense"``;
     the HIP v2 path for topk / router / quest with ``SEL.kernel_v2``; the HIP
     v1 per-row path otherwise (:790-804).  The sparse paths need S_q == S_k.  Returns
     ``(attn_output [B, S, H, D] contiguous, None)``.
@@ -480,6 +483,8 @@ def block_sparse_attention(module, query, key, value, attention_mask,
     is_prefill = Q > 1
     H, Hk = query.shape[1], key.shape[1]
 
+    if Q == 1 and (out := decode_attn(query, key, value, scaling)) is not None:
+        return out, None
     if SEL.mode == "dense" or Q == 1:
         ev = PROF.start("dense_sdpa") if is_prefill else None
         out = F.scaled_dot_product_attention(query, key, value, is_causal=Q > 1,
