@@ -160,12 +160,15 @@ int ugbsa_score_dump(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m, in
   dump.dump = 1;
   const uint16_t* q16 = static_cast<const uint16_t*>(q);
   const uint16_t* p16 = static_cast<const uint16_t*>(planes);
-  hipError_t e = ugbsa::launch_select(q16, sq_b, sq_h, sq_m, p16, B, H, Hk, M, N, D, dtype, mode, scaling,
-                                      k_b, rho_k + 1, 0, nullptr, nullptr, tile_score, st, &dump);
-  if (e != hipSuccess) return hip_result(e, "score_dump select");
-  return hip_result(ugbsa::launch_score_tau(q16, sq_b, sq_h, sq_m, p16, B, H, Hk, M, N, D, dtype, mode,
-                                            scaling, tau_hat, st),
-                    "score_dump tau");
+  // g and r hold the noise estimate's partial sums until the select launch
+  // writes them
+  hipError_t e = ugbsa::launch_score_tau(q16, sq_b, sq_h, sq_m, p16, B, H, Hk, M, N, D, dtype, mode,
+                                         scaling, g, r, tau_hat, st);
+  if (e != hipSuccess) return hip_result(e, "score_dump tau");
+  return hip_result(ugbsa::launch_select(q16, sq_b, sq_h, sq_m, p16, B, H, Hk, M, N, D, dtype, mode,
+                                         scaling, k_b, rho_k + 1, 0, nullptr, nullptr, tile_score,
+                                         st, &dump),
+                    "score_dump select");
 }
 
 int ugbsa_router(const float* sigma, int B, int H, int Qt, int grain, int rmode, float tau,

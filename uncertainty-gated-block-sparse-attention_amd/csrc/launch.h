@@ -77,11 +77,12 @@ struct RowsArgs {
 
 hipError_t launch_select_rows(const RowsArgs& a, hipStream_t stream);
 
-// Per-(b, h) score-noise estimate tau_hat of the score dump.
+// Per-(b, h) score-noise estimate tau_hat of the score dump; scratch_a and
+// scratch_b hold B * H * Qt floats each (the partial sums).
 hipError_t launch_score_tau(const uint16_t* q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
                             const uint16_t* planes, int B, int H, int Hk, int M, int N, int D,
-                            int elem, int mode, float scaling, float* tau_hat,
-                            hipStream_t stream);
+                            int elem, int mode, float scaling, float* scratch_a,
+                            float* scratch_b, float* tau_hat, hipStream_t stream);
 
 hipError_t launch_router(const float* sigma, int B, int H, int Qt, int grain, int rmode,
                          float tau, int64_t k_quant, int32_t* kv_idx, int k_base, int k_slots,

@@ -151,9 +151,10 @@ def record(query, key_states, scaling, block_m=64, sel=None, want_tile_score=Fal
     planes = sparse_attention.block_summary(key_states, mode)
     query = sparse_attention._contig_rows(query)
     f32 = dict(dtype=torch.float32, device=dev)
-    g, r, sigma, g_rho = (torch.empty(B, H, qt, **f32) for _ in range(4))
-    valid = torch.empty(qt, dtype=torch.uint8, device=dev)
-    tau = torch.empty(B, H, **f32)
+    # the shard's arrays side by side, so that one copy brings them to the host
+    cells = B * H * qt
+    flat = torch.empty(4 * cells + B * H + (qt + 3) // 4, **f32)
+    g, r, sigma, g_rho, tau, valid = flat.split([cells] * 4 + [B * H, (qt + 3) // 4])
     ts = torch.empty(B, H, qt, nb, **f32) if want_tile_score else None
     _capi.check(lib.ugbsa_score_dump(query.data_ptr(), *query.stride(), planes.data_ptr(),
                                      B, H, Hk, M, N, D, _capi.dtype_code(query.dtype), mode, float(scaling),
@@ -161,11 +162,13 @@ def record(query, key_states, scaling, block_m=64, sel=None, want_tile_score=Fal
                                      g_rho.data_ptr(), valid.data_ptr(), tau.data_ptr(),
                                      _capi.ptr(ts), _capi.stream_ptr(dev)),
                 "score dump")
+    host = flat.cpu().numpy()
+    stats = host[:4 * cells].reshape(4, B, H, qt)
     shard = {"n_blocks": int(nb), "mode_id": _mode_id(sel),
              "budget_blocks": int(sel.budget_blocks),
-             "g": g.cpu().numpy(), "r": r.cpu().numpy(), "sigma": sigma.cpu().numpy(),
-             "g_rho": g_rho.cpu().numpy(), "valid": valid.cpu().numpy().astype(bool),
-             "tau_hat": tau.cpu().numpy()}
+             "g": stats[0], "r": stats[1], "sigma": stats[2], "g_rho": stats[3],
+             "valid": host[4 * cells + B * H:].view("uint8")[:qt].astype(bool),
+             "tau_hat": host[4 * cells:4 * cells + B * H].reshape(B, H)}
     if want_tile_score:
         shard["tile_score"] = ts
     return shard
