@@ -1,0 +1,81 @@
+"""Attention calls of few tiles, where two or four wavefronts share a tile's list and merge."""
+
+import numpy as np
+import pytest
+import torch
+
+from block_attn import block_sparse_attn, block_sparse_attn_v2
+from oracle import attention as OA
+from parity import f32np
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+MAX_ABS, MEAN_ABS = 2e-2, 2e-3      # the bar of the attention tests
+
+
+def qkv(seed, B, H, Hk, M, D, dtype):
+    g = torch.Generator().manual_seed(seed)
+    return tuple(torch.randn(B, h, M, D, generator=g).to(dtype) for h in (H, Hk, Hk))
+
+
+def check(out, ref):
+    err = np.abs(f32np(out) - ref)
+    assert err.max() <= MAX_ABS and err.mean() <= MEAN_ABS, (err.max(), err.mean())
+
+
+# (H, M): 12 tiles and 72 (four wavefronts a tile), 360 (two), 720 (one); lists from none to every
+# visible block, so runs of no, one and several blocks, and one list in slot order (repeats)
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float16),
+                                     (128, torch.bfloat16), (128, torch.float16)])
+@pytest.mark.parametrize("H,M", [(4, 190), (4, 1150), (20, 1101), (40, 1150)])
+def test_tile_lists(hip_lib, D, dtype, H, M):
+    print(f"[case] split lists D={D} {dtype} H={H} M={M}", flush=True)
+    q, k, v = qkv(H + M + D, 1, H, H // 2, M, D, dtype)
+    nb = qt = (M + 63) // 64
+    g = torch.Generator().manual_seed(M)
+    kv = torch.full((1, H, qt, nb), nb, dtype=torch.int32)
+    for h in range(H):
+        for t in range(qt):
+            n = (h + t) % (t + 2)                       # 0 .. t + 1 blocks
+            pick = torch.randperm(t + 1, generator=g)[:n].to(torch.int32)
+            at = torch.randperm(nb, generator=g)[:n]    # sentinels between them
+            kv[0, h, t, at] = pick
+    if nb >= 5:
+        kv[0, 1, 4] = nb
+        kv[0, 1, 4, :5] = torch.tensor([3, 0, 3, 4, 0], dtype=torch.int32)
+    out = torch.full((1, H, M, D), float("nan"), dtype=dtype, device=DEV)
+    block_sparse_attn_v2(q.to(DEV), k.to(DEV), v.to(DEV), kv.to(DEV), D ** -0.5, out=out)
+    ref = OA.gathered_attention(f32np(q), f32np(k), f32np(v), kv.numpy(), D ** -0.5)
+    check(out, ref)
+    for h in range(min(H, 4)):
+        for t in range(qt):
+            if (h + t) % (t + 2) == 0 and (h, t) != (1, 4):
+                assert (out[0, h, 64 * t:64 * t + 64] == 0).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H,M", [(4, 190), (20, 1101)])
+def test_row_masks(hip_lib, D, H, M):
+    print(f"[case] split row masks D={D} H={H} M={M}", flush=True)
+    q, k, v = qkv(H + M + D, 1, H, H // 2, M, D, torch.bfloat16)
+    nb = (M + 63) // 64
+    g = torch.Generator().manual_seed(M)
+    rows = torch.arange(M)
+    keep = torch.rand(1, H, M, nb, generator=g) < 0.4
+    keep[0, :, rows, rows // 64] = True
+    out = block_sparse_attn(q.to(DEV), k.to(DEV), v.to(DEV), keep.to(DEV), D ** -0.5)
+    keep &= torch.arange(nb) <= (rows // 64)[:, None]
+    check(out, OA.keep_attention(f32np(q), f32np(k), f32np(v), keep.numpy(), D ** -0.5))
+
+
+def test_offsets_far_apart(hip_lib):
+    """Runs whose row maxima differ by hundreds of log2 units merge without overflow."""
+    D, H, M = 128, 4, 1150
+    q, k, v = qkv(7, 1, H, H, M, D, torch.bfloat16)
+    k[:, :, 640:704] *= 40.0
+    nb = qt = (M + 63) // 64
+    kv = torch.full((1, H, qt, nb), nb, dtype=torch.int32)
+    for t in range(qt):
+        kv[0, :, t, :t + 1] = torch.arange(t + 1, dtype=torch.int32)
+    out = block_sparse_attn_v2(q.to(DEV), k.to(DEV), v.to(DEV), kv.to(DEV), D ** -0.5)
+    check(out, OA.gathered_attention(f32np(q), f32np(k), f32np(v), kv.numpy(), D ** -0.5))

@@ -34,7 +34,8 @@
 // G query heads of one (b, KV head, t) are placed on the same XCD (workgroup
 // i runs on XCD i % 8), so their shared picks (sink, local, group needles)
 // hit the same L2; long contexts launch the units in generations
-// (attn_pipe.h, launch_attn_pipe).
+// (attn_pipe.h, launch_attn_pipe_t).  A call whose wavefronts all start at once
+// is not ranked (its two launches are 9 us of a 512-token layer).
 
 #include "common.h"
 #include "launch.h"
@@ -239,6 +240,40 @@ static bool uses_pipe(int D, int block_m) {
 }
 // Longest kv_idx row the pipelined kernel compacts into LDS.
 constexpr int kPipeMaxSlots = 16384;
+
+// Wavefronts of the pipelined kernel the chip holds at once: one per SIMD of
+// 256 CUs, two at head_dim 64.
+static int pipe_slots(int D) { return D == 64 ? 2048 : 1024; }
+
+// Wavefronts per 64-row tile.  A tile is a chain of its listed blocks, so a
+// call of few tiles, or of one round of tiles with long lists, leaves SIMDs idle
+// while the longest lists finish; two or four wavefronts then take a run of the
+// list each and merge.  Each costs a prologue and the merge, about 6 blocks of
+// a chain unsplit and 8 split (11-16 us against 1.8 us per block at head_dim
+// 128), so the rule compares (in blocks) the longest wavefront and the whole
+// work over the chip, plus a quarter of the longest for the ragged end, and
+// splits for at least 7 %.  Attention, us, 1 / 2 / 4 wavefronts (the rule's
+// choice first): head_dim 128, 28 heads, 8 blocks of 512 tokens 17.9 (4; 23.3,
+// 19.6), 16 of 1K 29.1 (2; 38.2, 40.5), 32 of 2K 63.6 (2; 69.0, 82.4), 64 of 4K
+// 138 (1; 152, 183); 8 heads, 32 of 2K 29.9 (4; 60.6, 40.4), 157 of 10K 230 (2;
+// 272, 240), 64 of 10K 144 (1; 155, 170); head_dim 64, 8 heads, 157 of 10K 147
+// (4; 249, 173), 16 heads, 32 of 8K 89 (1; 103, 103).
+static int attn_split(int64_t tiles, int Qt, int k_slots, int NB, int D, bool rowmask) {
+  if (NB > kGenBlocks || D > 128) return 1;
+  const int64_t most = k_slots < Qt ? k_slots : Qt;             // longest list
+  const double mean = most - 0.5 * most * (most - 1) / Qt;      // sum of min(t + 1, most) / Qt
+  int best = 1;
+  double best_t = 0.0;
+  for (int s = 1; s <= 4; s *= 2) {
+    if (s * pipe_wave_lds(D, 4, D != 128, k_slots, NB, rowmask) > 160 * 1024) break;
+    const double fixed = s == 1 ? 6.0 : 8.0;
+    const double longest = fixed + static_cast<double>(most) / s;
+    const double all = tiles * (fixed * s + mean) / pipe_slots(D);
+    const double t = (longest > all ? longest : all) + 0.25 * longest;
+    if (s == 1 || t < 0.93 * best_t) { best = s; best_t = t; }
+  }
+  return best;
+}
 
 hipError_t launch_attn_prepare(const uint16_t* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
                                const uint16_t* v, int64_t sv_b, int64_t sv_h, int64_t sv_n,
@@ -524,8 +559,10 @@ static hipError_t launch_attn_fwd_e(const uint16_t* q, int64_t sq_b, int64_t sq_
   if (uses_pipe(D, block_m)) {   // the pipelined kernel (its K/V operand layout is prepared)
     if (k_slots > kPipeMaxSlots) return hipErrorInvalidValue;
     const int NBk = (N + kBlock - 1) / kBlock;
+    const int64_t tiles = static_cast<int64_t>(B) * H * Qt;
+    const int split = attn_split(tiles, Qt, k_slots, NBk, D, rowmask != nullptr);
     const int32_t* tile_order = nullptr;
-    if (order_ws != nullptr) {
+    if (order_ws != nullptr && tiles * split > pipe_slots(D)) {   // else all start at once
       hipError_t e = launch_attn_tile_order(kv_idx, si_b, si_h, si_t, B, H, Qt, k_slots, NBk,
                                             order_ws, stream);
       if (e != hipSuccess) return e;
@@ -538,10 +575,10 @@ static hipError_t launch_attn_fwd_e(const uint16_t* q, int64_t sq_b, int64_t sq_
     if (D == 128)
       return launch_attn_pipe<E, 128, 4, false, false>(q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx,
                                           rowmask, si_b, si_h, si_t, B, H, Hk, M, N, Qt, k_slots,
-                                          scale, out, so_b, so_h, so_m, stream, tile_order);
+                                          scale, out, so_b, so_h, so_m, stream, tile_order, split);
     return launch_attn_pipe<E, 64, 4, true, true>(q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx,
                                        rowmask, si_b, si_h, si_t, B, H, Hk, M, N, Qt, k_slots,
-                                       scale, out, so_b, so_h, so_m, stream, tile_order);
+                                       scale, out, so_b, so_h, so_m, stream, tile_order, split);
   }
   // 32-row tiles: the older kernel (K read in place, V^T per block)
   if (block_m != 32) return hipErrorInvalidValue;

@@ -18,10 +18,10 @@ hipError_t launch_attn_pipe256(int elem, const uint16_t* q, int64_t sq_b, int64_
   if (elem == ElemF16::code)
     return launch_attn_pipe<ElemF16, 256, 4, true, true, true>(
         q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx, rowmask, si_b, si_h, si_t, B, H, Hk,
-        M, N, Qt, k_slots, scale, out, so_b, so_h, so_m, stream, tile_order);
+        M, N, Qt, k_slots, scale, out, so_b, so_h, so_m, stream, tile_order, 1);
   return launch_attn_pipe<ElemBf16, 256, 4, true, true, true>(
       q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx, rowmask, si_b, si_h, si_t, B, H, Hk, M,
-      N, Qt, k_slots, scale, out, so_b, so_h, so_m, stream, tile_order);
+      N, Qt, k_slots, scale, out, so_b, so_h, so_m, stream, tile_order, 1);
 }
 
 }  // namespace ugbsa

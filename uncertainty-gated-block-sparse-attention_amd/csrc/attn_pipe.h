@@ -45,6 +45,9 @@ namespace ugbsa {
 // 199 / 360, two with the row sums 186 / 339 (816 TFLOP/s).
 // The tile's kv_idx row is compacted into LDS once (visited blocks only), so
 // sentinel and invisible slots cost nothing in the loop.
+// SPLIT > 1 (head_dim 64 / 128, calls of few tiles): the workgroup's SPLIT
+// wavefronts all hold the tile's rows, each visits one run of its list, and
+// they merge (O, m, l) through LDS.
 // Per-wave LDS bytes of attn_fwd_pipe_kernel: Q fragments (QLDS), block
 // list, bitmap words and (with row masks) one mask per listed slot.
 __host__ __device__ inline int pipe_wave_lds(int D, int NT, bool qlds, int k_slots, int NB,
@@ -56,11 +59,18 @@ __host__ __device__ inline int pipe_wave_lds(int D, int NT, bool qlds, int k_slo
 }
 
 // Contexts of more than kGenBlocks key blocks run the attention units in
-// generations (launch_attn_pipe).
+// generations (launch_attn_pipe_t).
 constexpr int kGenBlocks = 512;
 
-template <typename E, int D, int NT, bool QLDS, bool SB, bool OA>
-__global__ __launch_bounds__(64 * (4 / NT), D == 64 ? 2 : 1) void attn_fwd_pipe_kernel(
+// LDS bytes of the merge of a tile's SPLIT wavefronts: their (m, l) and kMergeDt
+// 16-dim slices of their O^T at a time, as the lanes hold them.
+constexpr int kMergeDt = 4;
+__host__ __device__ constexpr int pipe_merge_lds(int NT, int split) {
+  return split == 1 ? 0 : split * NT * 64 * (kMergeDt * 16 + 8);
+}
+
+template <typename E, int D, int NT, bool QLDS, bool SB, bool OA, int SPLIT>
+__global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_fwd_pipe_kernel(
     const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
     const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
     const uint16_t* __restrict__ vt, const int32_t* __restrict__ kv_idx,
@@ -75,10 +85,14 @@ __global__ __launch_bounds__(64 * (4 / NT), D == 64 ? 2 : 1) void attn_fwd_pipe_
   // OA: O^T accumulates in AGPRs (a 64-row tile at head_dim 256 fills all
   // 256 of them), written only by the P.V MFMAs of the SB loop
   static_assert(!OA || SB, "AGPR accumulators are used by the single-set loop");
-  const int wave = threadIdx.x >> 6;
+  // (at head_dim 256 the merge spilled 200-600 bytes of O^T per lane)
+  static_assert(SPLIT == 1 || (NT == 4 && !OA), "a split tile's wavefronts hold all of its rows");
+  const int wave = SPLIT > 1 ? 0 : threadIdx.x >> 6;
+  const int part_id = SPLIT > 1 ? threadIdx.x >> 6 : 0;
   // dynamic LDS per wave: [Q fragments (QLDS)] [block list] [bitmap] [row masks]
   extern __shared__ __align__(16) unsigned char psm_all[];
-  unsigned char* psm = psm_all + wave * pipe_wave_lds(D, NT, QLDS, k_slots, NB, rowmask != nullptr);
+  unsigned char* psm = psm_all + (threadIdx.x >> 6) *
+                                     pipe_wave_lds(D, NT, QLDS, k_slots, NB, rowmask != nullptr);
   constexpr int QBYTES = QLDS ? NT * KS * 64 * 16 : 0;
   int32_t* blist = reinterpret_cast<int32_t*>(psm + QBYTES);
 
@@ -184,7 +198,7 @@ __global__ __launch_bounds__(64 * (4 / NT), D == 64 ? 2 : 1) void attn_fwd_pipe_
   // (Not with Q staged in LDS: at head_dim 256 it measured 1 % slower.)
   KSet ka, kb;
   VSet va, vb;
-  if constexpr (!QLDS) {
+  if constexpr (!QLDS && SPLIT == 1) {
     load_k(0, 0, ka);
     if constexpr (!SB) load_k(0, 1, kb);
     load_v(0, 0, va);
@@ -251,6 +265,13 @@ __global__ __launch_bounds__(64 * (4 / NT), D == 64 ? 2 : 1) void attn_fwd_pipe_
       pos = __shfl(at, 63, 64);
     }
     wave_lds_sync();
+  }
+
+  if constexpr (SPLIT > 1) {   // this wavefront's run of the tile's list
+    const int first = nv * part_id / SPLIT;
+    nv = nv * (part_id + 1) / SPLIT - first;
+    blist += first;
+    mlist += first;
   }
 
   // ---- Q tile: MFMA B operands held in registers ---------------------------
@@ -657,7 +678,7 @@ __global__ __launch_bounds__(64 * (4 / NT), D == 64 ? 2 : 1) void attn_fwd_pipe_
     };
     if (nv > 0) {
       const int b0 = uni(blk_raw(0));
-      if (QLDS || b0 != 0) {
+      if (QLDS || SPLIT > 1 || b0 != 0) {
         load_k(b0, 0, ka);
         load_v(b0, 0, va);
       }
@@ -725,7 +746,7 @@ __global__ __launch_bounds__(64 * (4 / NT), D == 64 ? 2 : 1) void attn_fwd_pipe_
     // V(u+1) outstanding at each step), so that the wait counts the compiler
     // derives for the loop hold for its first iteration as for the others
     const int b0 = uni(blk_raw(0));
-    if (QLDS || b0 != 0) {
+    if (QLDS || SPLIT > 1 || b0 != 0) {
       load_k(b0, 0, ka);
       load_k(b0, 1, kb);
       load_v(b0, 0, va);
@@ -750,9 +771,71 @@ __global__ __launch_bounds__(64 * (4 / NT), D == 64 ? 2 : 1) void attn_fwd_pipe_
     pv(vb);
   }
 
-  // ---- normalise and store ------------------------------------------------
   drain_o();
   uint16_t* ob = out + b * so_b + h * so_h;
+  if constexpr (SPLIT > 1) {
+    // ---- merge the tile's wavefronts through LDS, normalise and store --------
+    // Wavefront w finishes row sets [w NT / SPLIT, (w + 1) NT / SPLIT): every
+    // lane adds what the same lane of each wavefront holds of them, scaled to
+    // the largest of their offsets.  A run without blocks has m = -1e30, l = 0.
+    constexpr int RS = NT / SPLIT;
+    static_assert(RS * SPLIT == NT && DT % kMergeDt == 0, "whole row sets and passes");
+    f32x4* mo = reinterpret_cast<f32x4*>(psm_all);                 // [SPLIT][NT][kMergeDt][64]
+    float2* mml = reinterpret_cast<float2*>(mo + SPLIT * NT * kMergeDt * 64);
+    __syncthreads();           // lists and Q are read no more
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+      mml[(part_id * NT + nt) * 64 + lane] = make_float2(m[nt], l[nt]);
+    float f[RS][SPLIT], inv[RS];
+#pragma unroll
+    for (int ps = 0; ps < DT / kMergeDt; ++ps) {
+      if (ps > 0) __syncthreads();
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int j = 0; j < kMergeDt; ++j)
+          mo[((part_id * NT + nt) * kMergeDt + j) * 64 + lane] = o[ps * kMergeDt + j][nt];
+      __syncthreads();
+#pragma unroll
+      for (int rs = 0; rs < RS; ++rs) {
+        const int nt = part_id * RS + rs;
+        if (ps == 0) {
+          float mv[SPLIT], lv[SPLIT], mm = -1e30f, lt = 0.f;
+#pragma unroll
+          for (int w = 0; w < SPLIT; ++w) {
+            const float2 x = mml[(w * NT + nt) * 64 + lane];
+            mv[w] = x.x;
+            lv[w] = x.y;
+            mm = fmaxf(mm, mv[w]);
+          }
+#pragma unroll
+          for (int w = 0; w < SPLIT; ++w) {
+            f[rs][w] = __builtin_amdgcn_exp2f(mv[w] - mm);
+            lt += lv[w] * f[rs][w];
+          }
+          lt = quad_rows_sum(lt);
+          inv[rs] = lt > 0.f ? 1.0f / lt : 1.0f;
+        }
+        const int row = row0 + 16 * nt + r16;
+#pragma unroll
+        for (int j = 0; j < kMergeDt; ++j) {
+          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int w = 0; w < SPLIT; ++w)
+            acc += mo[((w * NT + nt) * kMergeDt + j) * 64 + lane] * f[rs][w];
+          if (row < M) {
+            const uint32_t w0 = E::pack2(acc[0] * inv[rs], acc[1] * inv[rs]);
+            const uint32_t w1 = E::pack2(acc[2] * inv[rs], acc[3] * inv[rs]);
+            *reinterpret_cast<uint2*>(ob + row * so_m + 16 * (ps * kMergeDt + j) + 4 * g4) =
+                make_uint2(w0, w1);
+          }
+        }
+      }
+    }
+    return;
+  }
+
+  // ---- normalise and store ------------------------------------------------
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     float lt = l[nt];
@@ -800,26 +883,27 @@ static int resident_workgroups(Kern kern, int threads, size_t lds) {
 template <int D>
 constexpr int gen_waves() { return D > 128 ? 1 : 3; }
 
-// tile_order (optional): the (b, t) tiles heaviest first (attn_tile_order);
-// it enables the generations above.  Without it, one launch with tiles by t
-// descending.
-template <typename E, int D, int NT, bool QLDS, bool SB, bool OA = false>
-static hipError_t launch_attn_pipe(const uint16_t* q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
-                                   const uint16_t* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
-                                   const uint16_t* vt, const int32_t* kv_idx,
-                                   const uint64_t* rowmask, int64_t si_b, int64_t si_h,
-                                   int64_t si_t, int B, int H, int Hk, int M, int N, int Qt,
-                                   int k_slots, float scale, uint16_t* out, int64_t so_b,
-                                   int64_t so_h, int64_t so_m, hipStream_t stream,
-                                   const int32_t* tile_order = nullptr) {
+// One launch (or the generations of one call): tile_order (optional) holds the
+// (b, t) tiles heaviest first (attn_tile_order) and enables the generations
+// above; without it, one launch with tiles by t descending.
+template <typename E, int D, int NT, bool QLDS, bool SB, bool OA, int SPLIT>
+static hipError_t launch_attn_pipe_t(const uint16_t* q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
+                                     const uint16_t* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
+                                     const uint16_t* vt, const int32_t* kv_idx,
+                                     const uint64_t* rowmask, int64_t si_b, int64_t si_h,
+                                     int64_t si_t, int B, int H, int Hk, int M, int N, int Qt,
+                                     int k_slots, float scale, uint16_t* out, int64_t so_b,
+                                     int64_t so_h, int64_t so_m, hipStream_t stream,
+                                     const int32_t* tile_order) {
   const int NB = (N + kBlock - 1) / kBlock;
   const int grp = H / Hk;
   const int units = B * Hk * Qt;
-  constexpr int WPT = 4 / NT;
-  const size_t lds = static_cast<size_t>(WPT) *
-                     pipe_wave_lds(D, NT, QLDS, k_slots, NB, rowmask != nullptr);
+  constexpr int WPT = 4 / NT * SPLIT;
+  size_t lds = static_cast<size_t>(WPT) *
+               pipe_wave_lds(D, NT, QLDS, k_slots, NB, rowmask != nullptr);
+  if (lds < static_cast<size_t>(pipe_merge_lds(NT, SPLIT))) lds = pipe_merge_lds(NT, SPLIT);
   if (lds > 160 * 1024) return hipErrorInvalidConfiguration;
-  auto kern = attn_fwd_pipe_kernel<E, D, NT, QLDS, SB, OA>;
+  auto kern = attn_fwd_pipe_kernel<E, D, NT, QLDS, SB, OA, SPLIT>;
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -845,6 +929,28 @@ static hipError_t launch_attn_pipe(const uint16_t* q, int64_t sq_b, int64_t sq_h
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+// split: wavefronts per 64-row tile (attn_split).
+template <typename E, int D, int NT, bool QLDS, bool SB, bool OA = false>
+static hipError_t launch_attn_pipe(const uint16_t* q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
+                                   const uint16_t* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
+                                   const uint16_t* vt, const int32_t* kv_idx,
+                                   const uint64_t* rowmask, int64_t si_b, int64_t si_h,
+                                   int64_t si_t, int B, int H, int Hk, int M, int N, int Qt,
+                                   int k_slots, float scale, uint16_t* out, int64_t so_b,
+                                   int64_t so_h, int64_t so_m, hipStream_t stream,
+                                   const int32_t* tile_order, int split) {
+#define UGBSA_PIPE(S_)                                                                          \
+  return launch_attn_pipe_t<E, D, NT, QLDS, SB, OA, S_>(                                       \
+      q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx, rowmask, si_b, si_h, si_t, B, H, Hk, \
+      M, N, Qt, k_slots, scale, out, so_b, so_h, so_m, stream, tile_order)
+  if constexpr (!OA) {
+    if (split == 4) UGBSA_PIPE(4);
+    if (split == 2) UGBSA_PIPE(2);
+  }
+  UGBSA_PIPE(1);
+#undef UGBSA_PIPE
 }
 
 
