@@ -74,6 +74,13 @@ int ugbsa_block_summary(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
                         int B, int Hk, int N, int D, int dtype, int mode, void* planes,
                         void* stream);
 
+/* ugbsa_block_summary in mean mode, and the block means the planes hold rounded
+ * to dtype, repeated for the query heads: means [B, H, NB, D] (the v1
+ * selector's k_pool_at, src/sparse_attention.py:230-232). */
+int ugbsa_block_summary_means(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
+                              int64_t sk_d, int B, int H, int Hk, int N, int D, int dtype,
+                              void* planes, void* means, void* stream);
+
 /* Kernel 2 — fused per-Q-tile block scoring, tile max-pool, visibility,
  * sink/self forcing, top-k_slots and (if sigma != NULL) the sigma margin.
  * Replaces src/sparse_attention.py:623-707 of _block_select_kv_idx_v2

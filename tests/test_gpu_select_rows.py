@@ -1,10 +1,15 @@
 """Per-row selection at the edges of its register layouts (1, 2, 4, .. blocks per lane), with ties,
-NaN scores and margins at other ranks than the budget, against the oracle on the kernel's scores."""
+NaN scores and margins at other ranks than the budget, against the oracle on the kernel's scores;
+the lists and row masks made of keep masks, and the cached block means."""
 
+import numpy as np
 import pytest
 import torch
 
+import _capi
 import sparse_attention as sa
+from block_attn import keep_kv_idx
+from oracle import attention as OA
 from test_gpu_select_v1 import check_on_kernel_scores, make_sel
 
 pytestmark = pytest.mark.gpu
@@ -58,3 +63,41 @@ def test_nan_and_infinite_scores(hip_lib):
     for mode, kw in (("quest", dict(budget_blocks=16)),
                      ("router", dict(budget_blocks=12, router_score="quest"))):
         check(mode, kw, q, k)
+
+
+# 1-, 4- and 8-byte words, one block, part of a 64-block step, one and several 1024-block sections
+@pytest.mark.parametrize("nb", [1, 5, 64, 100, 132, 256, 260, 1024, 1025, 1032, 2056])
+@pytest.mark.parametrize("block_m", [64, 32])
+def test_keep_lists(hip_lib, nb, block_m):
+    print(f"[case] keep lists nb={nb} block_m={block_m}", flush=True)
+    g = torch.Generator().manual_seed(nb)
+    M = 150                                             # a ragged last tile
+    keep = torch.rand(2, 3, M, nb, generator=g) < 0.02
+    keep[0, 1, 64:128] = False                          # a tile that keeps nothing
+    want, want_max = OA.compute_kv_idx(keep.numpy(), block_m)
+    odd = torch.empty(keep.numel() + 1, dtype=torch.bool, device=DEV)[1:].view(keep.shape)
+    odd.copy_(keep)                                     # no word of it is aligned
+    for dev in (keep.to(DEV), odd):
+        kv, rm, most = keep_kv_idx(dev, block_m)
+        assert most == want_max
+        got = kv.cpu().numpy()
+        assert np.array_equal(got[..., :most], want) and (got[..., most:] == nb).all()
+        masks = rm.cpu().numpy().view(np.uint64)
+        for t in range(got.shape[2]):
+            rows = keep[:, :, t * block_m:(t + 1) * block_m].numpy()
+            bits = (rows.astype(np.uint64) << np.arange(rows.shape[2], dtype=np.uint64)[:, None]).sum(2)
+            pad = np.concatenate([bits, np.zeros_like(bits[..., :1])], -1)       # the sentinel: none
+            assert np.array_equal(masks[:, :, t], np.take_along_axis(pad, got[:, :, t], -1))
+
+
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16), (256, torch.bfloat16)])
+def test_cached_block_means(hip_lib, D, dtype):
+    """k_pool_at holds the means of the summary planes in the model's dtype, once per query head."""
+    g = torch.Generator().manual_seed(D)
+    q = torch.randn(2, 4, 300, D, generator=g).to(dtype).to(DEV)
+    k = torch.randn(2, 2, 300, D, generator=g).to(dtype).to(DEV)
+    sel = make_sel(mode="topk")
+    sa.select_mask_v1(q, k, 0.1, sel=sel, layer_idx=7)
+    planes = sa.block_summary(k, _capi.MODE_MEAN)
+    want = sa.block_means(planes, 2, 2, 5, D).repeat_interleave(2, dim=1).to(dtype)
+    assert torch.equal(sel.k_pool_at[7], want)

@@ -34,6 +34,8 @@ SIGNATURES = {
     "ugbsa_last_error": (ctypes.c_char_p, []),
     "ugbsa_summary_elems": (_i64, [_i, _i, _i, _i, _i]),
     "ugbsa_block_summary": (_i, [_p, _i64, _i64, _i64, _i64, _i, _i, _i, _i, _i, _i, _p, _p]),
+    "ugbsa_block_summary_means": (_i, [_p, _i64, _i64, _i64, _i64, _i, _i, _i, _i, _i, _i, _p, _p,
+                                       _p]),
     "ugbsa_select": (_i, [_p, _i64, _i64, _i64, _i64, _p, _i, _i, _i, _i, _i, _i, _i, _i,
                           _f, _i, _i, _i, _p, _p, _p, _p]),
     "ugbsa_score_dump": (_i, [_p, _i64, _i64, _i64, _i64, _p, _i, _i, _i, _i, _i, _i, _i, _i,

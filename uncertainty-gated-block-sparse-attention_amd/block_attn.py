@@ -143,13 +143,8 @@ def decode_attn(q, k, v, scale):
     return out
 
 
-def keep_kv_idx(keep, block_m=64, want_rowmask=True):
-    """HIP compaction of a device keep mask [B, H, M, NB] (bool).
-
-    Returns (kv_idx [B, H, Qt, NB] int32 ascending and NB-padded, rowmask
-    [B, H, Qt, NB] int64 — bit r set where tile row r keeps the listed block —
-    or None, MAX_KEPT).  Synchronises once for MAX_KEPT, as the reference.
-    """
+def _keep_lists(keep, block_m, want_rowmask):
+    """(kv_idx, rowmask or None, counts) of ``ugbsa_keep_kv_idx``, on the device."""
     assert keep.is_cuda and keep.dtype == torch.bool and keep.dim() == 4
     keep = keep.contiguous()
     B, H, M, NB = keep.shape
@@ -161,8 +156,27 @@ def keep_kv_idx(keep, block_m=64, want_rowmask=True):
                                               _capi.ptr(rm), counts.data_ptr(),
                                               _capi.stream_ptr(keep.device)),
                 "keep_kv_idx")
+    return kv, rm, counts
+
+
+def keep_kv_idx(keep, block_m=64, want_rowmask=True):
+    """HIP compaction of a device keep mask [B, H, M, NB] (bool).
+
+    Returns (kv_idx [B, H, Qt, NB] int32 ascending and NB-padded, rowmask
+    [B, H, Qt, NB] int64 — bit r set where tile row r keeps the listed block —
+    or None, MAX_KEPT).  Synchronises once for MAX_KEPT, as the reference.
+    """
+    kv, rm, counts = _keep_lists(keep, block_m, want_rowmask)
     max_kept = max(1, int(counts.max().item()))
     return kv, rm, max_kept
+
+
+# The row-masked attention takes the lists NB wide, without asking the device for
+# the longest one (40 us of host time a call), while a 64-row tile's list and
+# masks, 12 bytes a slot in LDS, leave every CU its eight wavefronts at head_dim
+# 64 (four at 128 and 256); the 32-row tile kernel walks every slot, so there
+# the longest list is worth a synchronisation.
+_ROWS_LIST_BLOCKS = 1024
 
 
 def block_sparse_attn(q, k, v, keep, scale, block_n=64, block_m=64,
@@ -184,7 +198,11 @@ def block_sparse_attn(q, k, v, keep, scale, block_n=64, block_m=64,
     Hk, N = k.shape[1], k.shape[2]
     assert H % Hk == 0, "query heads must be a multiple of KV heads"
     assert tuple(keep.shape[:3]) == (B, H, M), "keep [B, H, M, NB] expected"
-    kv, rm, max_kept = keep_kv_idx(keep, block_m)
+    if block_m == 64 and keep.shape[3] <= _ROWS_LIST_BLOCKS:
+        kv, rm, _ = _keep_lists(keep, block_m, True)
+        max_kept = keep.shape[3]
+    else:
+        kv, rm, max_kept = keep_kv_idx(keep, block_m)
     q = _operand("q", q)
     k = _operand("k", k, q.dtype)
     v = _operand("v", v, q.dtype)

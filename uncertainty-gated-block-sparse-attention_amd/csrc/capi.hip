@@ -83,9 +83,9 @@ int64_t ugbsa_attn_workspace_elems(int B, int Hk, int N, int D) {
   return kv_copy_elems(B, Hk, N, D) + sched;
 }
 
-int ugbsa_block_summary(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n, int64_t sk_d,
-                        int B, int Hk, int N, int D, int dtype, int mode, void* planes,
-                        void* stream) {
+static int block_summary_impl(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
+                              int64_t sk_d, int B, int Hk, int N, int D, int dtype, int mode,
+                              void* planes, void* pool, int rep, void* stream) {
   int rc = check_dims(B, Hk, Hk, D, dtype);
   if (rc) return rc;
   if ((rc = check_bf16_operand("k", k, sk_b, sk_h, sk_n, sk_d))) return rc;
@@ -97,8 +97,26 @@ int ugbsa_block_summary(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
   if (!aligned16(planes)) return fail(UGBSA_ELAYOUT, "planes must be 16-byte aligned");
   return hip_result(ugbsa::launch_block_summary(static_cast<const uint16_t*>(k), sk_b, sk_h, sk_n, B, Hk, N, D,
                                                 dtype, mode, static_cast<uint16_t*>(planes),
-                                                static_cast<hipStream_t>(stream)),
+                                                static_cast<hipStream_t>(stream),
+                                                static_cast<uint16_t*>(pool), rep),
                     "block_summary");
+}
+
+int ugbsa_block_summary(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n, int64_t sk_d,
+                        int B, int Hk, int N, int D, int dtype, int mode, void* planes,
+                        void* stream) {
+  return block_summary_impl(k, sk_b, sk_h, sk_n, sk_d, B, Hk, N, D, dtype, mode, planes, nullptr,
+                            1, stream);
+}
+
+int ugbsa_block_summary_means(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
+                              int64_t sk_d, int B, int H, int Hk, int N, int D, int dtype,
+                              void* planes, void* means, void* stream) {
+  int rc = check_dims(B, H, Hk, D, dtype);
+  if (rc) return rc;
+  if (means == nullptr) return fail(UGBSA_EARG, "means is null");
+  return block_summary_impl(k, sk_b, sk_h, sk_n, sk_d, B, Hk, N, D, dtype, UGBSA_MODE_MEAN, planes,
+                            means, H / Hk, stream);
 }
 
 int ugbsa_select(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m, int64_t sq_d,

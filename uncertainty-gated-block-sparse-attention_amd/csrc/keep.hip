@@ -9,95 +9,107 @@
 // — the per-row keep test of the reference kernel (:87-103), read by the
 // attention kernels once per block instead of once per row.
 //
-// One wavefront per tile.  When rows are a multiple of 8 bytes (NB % 8 == 0,
-// mask 8-byte aligned)
-// a lane owns 8 consecutive blocks of each 512-block span and reads them as
-// one 8-byte word per row (a row's span is one coalesced 512-byte read), ORs
-// the row bits into 8 masks, and a wavefront prefix sum over the lanes'
-// counts places the kept blocks in ascending order.  Otherwise 64 blocks at
-// a time, one block per lane, with a ballot compaction.
+// One workgroup per tile, its four wavefronts a quarter of the tile's rows
+// each: a lane owns WB consecutive blocks (one WB-byte word per row, a quarter
+// tile's words requested together) and leaves its rows' bits of each block in
+// LDS, a fourth of the block's mask.  Then the workgroup compacts the section
+// 256 blocks at a time.  Latency-bound at the per-row lengths seen (64 to 512
+// blocks): a wavefront per tile, 8 rows at a time, took 23 us for 28 x 64 tiles
+// of 64 blocks, where 56 of its 64 lanes had no word, and 39 us for 8 x 157
+// tiles of 157 blocks a byte at a time; now 14 and 22 us.
 #include "common.h"
 #include "launch.h"
 
 namespace ugbsa {
 
-__global__ __launch_bounds__(256) void keep_kv_idx_kernel(
-    const uint8_t* __restrict__ keep, int B, int H, int M, int NB, int block_m, int Qt,
+constexpr int kKeepWaves = 4;
+constexpr int kKeepSection = 1024;    // blocks whose masks LDS holds at once
+
+// WB bytes (blocks) per lane and row: 8 or 4 where rows and the mask are
+// multiples of it and the row is long enough to give most lanes a word, else 1.
+template <int WB>
+__global__ __launch_bounds__(64 * kKeepWaves) void keep_kv_idx_kernel(
+    const uint8_t* __restrict__ keep, int M, int NB, int block_m, int Qt,
     int32_t* __restrict__ kv_idx, uint64_t* __restrict__ rowmask, int32_t* __restrict__ counts) {
-  const int lane = threadIdx.x & 63;
-  const int64_t unit = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (unit >= static_cast<int64_t>(B) * H * Qt) return;
+  constexpr int RW = 64 / kKeepWaves;    // mask bits per wavefront
+  __shared__ __align__(8) uint16_t s_mask[kKeepSection][kKeepWaves];   // one uint64 per block
+  __shared__ int s_cnt[kKeepWaves];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t unit = blockIdx.x;
   const int64_t bh = unit / Qt;
   const int t = static_cast<int>(unit % Qt);
   const int rows = min(block_m, M - t * block_m);
-  const uint8_t* kb = keep + (bh * M + static_cast<int64_t>(t) * block_m) * NB;
+  const int r0 = wave * RW;              // wavefronts past block_m have no rows
+  const uint8_t* kb = keep + (bh * M + static_cast<int64_t>(t) * block_m + r0) * NB;
   int32_t* out = kv_idx + unit * NB;
   uint64_t* rm = rowmask != nullptr ? rowmask + unit * NB : nullptr;
   const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   int cnt = 0;
-  if ((NB & 7) == 0 && (reinterpret_cast<uintptr_t>(keep) & 7) == 0) {
-    for (int base = 0; base < NB; base += 512) {
-      const int b0 = base + 8 * lane;
-      uint64_t mk[8] = {0ull, 0ull, 0ull, 0ull, 0ull, 0ull, 0ull, 0ull};
-      if (b0 < NB) {
-        const uint64_t* src = reinterpret_cast<const uint64_t*>(kb + b0);
-        const int64_t stride = NB / 8;
-        for (int r0 = 0; r0 < rows; r0 += 8) {
-          uint64_t w[8];
+  for (int base = 0; base < NB; base += kKeepSection) {
+    const int n = min(kKeepSection, NB - base);
+    if (base > 0) __syncthreads();       // the section before is compacted
+    for (int c = WB * lane; c < n; c += 64 * WB) {
+      uint32_t mk[WB];
 #pragma unroll
-          for (int j = 0; j < 8; ++j) w[j] = r0 + j < rows ? src[(r0 + j) * stride] : 0ull;
+      for (int i = 0; i < WB; ++i) mk[i] = 0u;
+      uint64_t w[RW];
 #pragma unroll
-          for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-              mk[i] |= static_cast<uint64_t>(((w[j] >> (8 * i)) & 0xFFull) != 0) << (r0 + j);
+      for (int r = 0; r < RW; ++r) {
+        const uint8_t* src = kb + static_cast<int64_t>(r) * NB + base + c;
+        w[r] = 0ull;
+        if (r0 + r < rows) {
+          if constexpr (WB == 8) w[r] = *reinterpret_cast<const uint64_t*>(src);
+          else if constexpr (WB == 4) w[r] = *reinterpret_cast<const uint32_t*>(src);
+          else w[r] = *src;
         }
       }
-      int mine = 0;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) mine += mk[i] != 0ull;
-      int pos = cnt + static_cast<int>(wave_excl_scan(static_cast<uint32_t>(mine), lane));
+      for (int r = 0; r < RW; ++r)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (mk[i] != 0ull) {
-          out[pos] = b0 + i;
-          if (rm != nullptr) rm[pos] = mk[i];
-          ++pos;
-        }
+        for (int i = 0; i < WB; ++i)
+          mk[i] |= static_cast<uint32_t>(((w[r] >> (8 * i)) & 0xFFull) != 0) << r;
+#pragma unroll
+      for (int i = 0; i < WB; ++i) s_mask[c + i][wave] = static_cast<uint16_t>(mk[i]);
+    }
+    __syncthreads();
+    for (int c = 0; c < n; c += 64 * kKeepWaves) {
+      const int i = c + threadIdx.x;
+      const uint64_t mask = i < n ? *reinterpret_cast<const uint64_t*>(s_mask[i]) : 0ull;
+      const uint64_t bal = __ballot(mask != 0ull);
+      if (c > 0) __syncthreads();        // the counts of the step before are read
+      if (lane == 0) s_cnt[wave] = __popcll(bal);
+      __syncthreads();
+      int pos = cnt + __popcll(bal & lt_mask);
+#pragma unroll
+      for (int v = 0; v < kKeepWaves; ++v) {
+        pos += v < wave ? s_cnt[v] : 0;
+        cnt += s_cnt[v];
       }
-      cnt = __shfl(pos, 63, 64);
+      if (mask != 0ull) {
+        out[pos] = base + i;
+        if (rm != nullptr) rm[pos] = mask;
+      }
     }
-  } else {
-  for (int base = 0; base < NB; base += 64) {
-    const int blk = base + lane;
-    uint64_t mask = 0;
-    if (blk < NB)
-      for (int r = 0; r < rows; ++r)
-        mask |= static_cast<uint64_t>(kb[static_cast<int64_t>(r) * NB + blk] != 0) << r;
-    const bool ok = mask != 0;
-    const uint64_t bal = __ballot(ok);
-    if (ok) {
-      const int pos = cnt + __popcll(bal & lt_mask);
-      out[pos] = blk;
-      if (rm != nullptr) rm[pos] = mask;
-    }
-    cnt += __popcll(bal);
   }
-  }
-  for (int s = cnt + lane; s < NB; s += 64) {
+  for (int s = cnt + threadIdx.x; s < NB; s += 64 * kKeepWaves) {
     out[s] = NB;
     if (rm != nullptr) rm[s] = 0ull;
   }
-  if (lane == 0) counts[unit] = cnt;
+  if (threadIdx.x == 0) counts[unit] = cnt;
 }
 
 hipError_t launch_keep_kv_idx(const uint8_t* keep, int B, int H, int M, int NB, int block_m,
                               int32_t* kv_idx, uint64_t* rowmask, int32_t* counts,
                               hipStream_t stream) {
   const int Qt = (M + block_m - 1) / block_m;
-  const int64_t waves = static_cast<int64_t>(B) * H * Qt;
-  keep_kv_idx_kernel<<<dim3(static_cast<unsigned>((waves + 3) / 4)), 256, 0, stream>>>(
-      keep, B, H, M, NB, block_m, Qt, kv_idx, rowmask, counts);
+  const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(B) * H * Qt));
+  const uintptr_t at = reinterpret_cast<uintptr_t>(keep);
+  if (NB % 8 == 0 && at % 8 == 0 && NB >= 256)
+    keep_kv_idx_kernel<8><<<grid, 64 * kKeepWaves, 0, stream>>>(keep, M, NB, block_m, Qt, kv_idx, rowmask, counts);
+  else if (NB % 4 == 0 && at % 4 == 0 && NB >= 128)
+    keep_kv_idx_kernel<4><<<grid, 64 * kKeepWaves, 0, stream>>>(keep, M, NB, block_m, Qt, kv_idx, rowmask, counts);
+  else
+    keep_kv_idx_kernel<1><<<grid, 64 * kKeepWaves, 0, stream>>>(keep, M, NB, block_m, Qt, kv_idx, rowmask, counts);
   return hipGetLastError();
 }
 

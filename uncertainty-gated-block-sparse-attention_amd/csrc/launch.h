@@ -28,9 +28,11 @@ constexpr int kMaxSlots = 512;
 
 // elem: the 16-bit element format of the call's tensors (ElemBf16::code 0 or
 // ElemF16::code 1, the C ABI's UGBSA_DTYPE_* values).
+// pool (mean mode, or null): the block means in K's format, [B, Hk * rep, NB, D].
 hipError_t launch_block_summary(const uint16_t* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
                                 int B, int Hk, int N, int D, int elem, int mode,
-                                uint16_t* planes, hipStream_t stream);
+                                uint16_t* planes, hipStream_t stream, uint16_t* pool = nullptr,
+                                int rep = 1);
 
 // Extra modes of the selection kernel.
 //  dump != 0: per-tile order statistics of the unforced tile scores, ranked

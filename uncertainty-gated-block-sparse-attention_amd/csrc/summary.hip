@@ -28,7 +28,8 @@ namespace ugbsa {
 template <int D, typename E>
 __global__ __launch_bounds__(256) void block_summary_kernel(
     const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
-    int B, int Hk, int N, int NB, int mode, uint16_t* __restrict__ planes) {
+    int B, int Hk, int N, int NB, int mode, uint16_t* __restrict__ planes,
+    uint16_t* __restrict__ pool, int rep) {
   constexpr int CH = D / 8;        // 16-byte chunks per row
   constexpr int RG = 256 / CH;     // row groups
   constexpr int RPG = kBlock / RG; // rows per group
@@ -96,8 +97,16 @@ __global__ __launch_bounds__(256) void block_summary_kernel(
     uint16_t* out = planes + bid * 2 * D;
     const float x = ldexpf(mean, e);                   // exact
     const uint16_t hi = ElemF16::from_f32(x);
+    const uint16_t lo = ElemF16::from_f32(x - ElemF16::to_f32(hi));
     out[d] = hi;
-    out[D + d] = ElemF16::from_f32(x - ElemF16::to_f32(hi));
+    out[D + d] = lo;
+    if (pool != nullptr) {
+      // the mean the planes hold, in K's format, once per query head
+      const float m = (ElemF16::to_f32(hi) + ElemF16::to_f32(lo)) * ldexpf(1.0f, -e);
+      const uint16_t m16 = static_cast<uint16_t>(E::pack2(m, 0.f) & 0xFFFFu);
+      for (int r = 0; r < rep; ++r)
+        pool[(((static_cast<int64_t>(b) * Hk + h) * rep + r) * NB + blk) * D + d] = m16;
+    }
   }
   if (threadIdx.x == 0) {
     float* descale = reinterpret_cast<float*>(planes + static_cast<int64_t>(B) * Hk * NB * 2 * D);
@@ -108,18 +117,19 @@ __global__ __launch_bounds__(256) void block_summary_kernel(
 template <typename E>
 static hipError_t launch_block_summary_e(const uint16_t* k, int64_t sk_b, int64_t sk_h,
                                          int64_t sk_n, int B, int Hk, int N, int D, int mode,
-                                         uint16_t* planes, hipStream_t stream) {
+                                         uint16_t* planes, uint16_t* pool, int rep,
+                                         hipStream_t stream) {
   const int NB = (N + kBlock - 1) / kBlock;
   dim3 grid(NB, Hk, B);
   switch (D) {
     case 64:
-      block_summary_kernel<64, E><<<grid, 256, 0, stream>>>(k, sk_b, sk_h, sk_n, B, Hk, N, NB, mode, planes);
+      block_summary_kernel<64, E><<<grid, 256, 0, stream>>>(k, sk_b, sk_h, sk_n, B, Hk, N, NB, mode, planes, pool, rep);
       break;
     case 128:
-      block_summary_kernel<128, E><<<grid, 256, 0, stream>>>(k, sk_b, sk_h, sk_n, B, Hk, N, NB, mode, planes);
+      block_summary_kernel<128, E><<<grid, 256, 0, stream>>>(k, sk_b, sk_h, sk_n, B, Hk, N, NB, mode, planes, pool, rep);
       break;
     case 256:
-      block_summary_kernel<256, E><<<grid, 256, 0, stream>>>(k, sk_b, sk_h, sk_n, B, Hk, N, NB, mode, planes);
+      block_summary_kernel<256, E><<<grid, 256, 0, stream>>>(k, sk_b, sk_h, sk_n, B, Hk, N, NB, mode, planes, pool, rep);
       break;
     default:
       return hipErrorInvalidValue;
@@ -129,10 +139,11 @@ static hipError_t launch_block_summary_e(const uint16_t* k, int64_t sk_b, int64_
 
 hipError_t launch_block_summary(const uint16_t* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
                                 int B, int Hk, int N, int D, int elem, int mode,
-                                uint16_t* planes, hipStream_t stream) {
+                                uint16_t* planes, hipStream_t stream, uint16_t* pool,
+                                int rep) {
   if (elem == ElemF16::code)
-    return launch_block_summary_e<ElemF16>(k, sk_b, sk_h, sk_n, B, Hk, N, D, mode, planes, stream);
-  return launch_block_summary_e<ElemBf16>(k, sk_b, sk_h, sk_n, B, Hk, N, D, mode, planes, stream);
+    return launch_block_summary_e<ElemF16>(k, sk_b, sk_h, sk_n, B, Hk, N, D, mode, planes, pool, rep, stream);
+  return launch_block_summary_e<ElemBf16>(k, sk_b, sk_h, sk_n, B, Hk, N, D, mode, planes, pool, rep, stream);
 }
 
 }  // namespace ugbsa

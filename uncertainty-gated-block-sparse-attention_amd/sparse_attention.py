@@ -218,16 +218,24 @@ def select_v2(query, key_states, scaling, block_m=64, sel: Selector = None,
     return res
 
 
-def block_summary(key_states, mode):
+def block_summary(key_states, mode, means=None):
     """Kernel 1: the K-block summaries of ``mode`` (``_capi.MODE_QUEST`` or
     ``_capi.MODE_MEAN``) as one flat buffer in K's dtype, on the current stream:
     Quest [B, Hk, NB, 2, D] (K-max, K-min); mean the fp16 planes [B, Hk, NB, 2, D]
-    then the fp32 block scales [B, Hk, NB] (``block_means`` decodes them)."""
+    then the fp32 block scales [B, Hk, NB] (``block_means`` decodes them).
+    ``means`` (mean mode): [B, H, NB, D] in K's dtype, filled with those means
+    repeated for the query heads."""
     B, Hk, N, D = key_states.shape
     lib = _capi.lib()
     key_states = _contig_rows(key_states)
     planes = torch.empty(lib.ugbsa_summary_elems(B, Hk, N, D, mode), dtype=key_states.dtype,
                          device=key_states.device)
+    if means is not None:
+        _capi.check(lib.ugbsa_block_summary_means(
+            key_states.data_ptr(), *key_states.stride(), B, means.shape[1], Hk, N, D,
+            _capi.dtype_code(key_states.dtype), planes.data_ptr(), means.data_ptr(),
+            _capi.stream_ptr(key_states.device)), "block summary")
+        return planes
     _capi.check(lib.ugbsa_block_summary(key_states.data_ptr(), *key_states.stride(), B, Hk, N, D,
                                         _capi.dtype_code(key_states.dtype), mode, planes.data_ptr(),
                                         _capi.stream_ptr(key_states.device)),
@@ -318,11 +326,12 @@ def select_mask_v1(query, key_states, scaling, sel: Selector = None, want_scores
     query = _contig_rows(query)
     nb = (N + BLOCK - 1) // BLOCK
     mode = _capi.MODE_QUEST if use_quest(sel) else _capi.MODE_MEAN
-    planes = block_summary(key_states, mode)
+    means = None
     if mode == _capi.MODE_MEAN and M > 1 and layer_idx is not None:
         # the mean K of each block, repeat_kv'd, cached for later planners (:230-232)
-        kp = block_means(planes, B, Hk, nb, D).repeat_interleave(H // Hk, dim=1)
-        sel.k_pool_at[layer_idx] = kp.to(query.dtype)
+        means = torch.empty(B, H, nb, D, dtype=query.dtype, device=dev)
+        sel.k_pool_at[layer_idx] = means
+    planes = block_summary(key_states, mode, means)
     k_bud = min(int(max(min(sel.k_max, sel.budget_blocks), sel.k_min)), nb)
     router = sel.mode == "router"
     k_eff = max(1, min(int(sel.budget_blocks), nb - 1)) if router else 0
