@@ -69,7 +69,7 @@ __host__ __device__ constexpr int pipe_merge_lds(int NT, int split) {
   return split == 1 ? 0 : split * NT * 64 * (kMergeDt * 16 + 8);
 }
 
-template <typename E, int D, int NT, bool QLDS, bool SB, bool OA, int SPLIT>
+template <typename E, int D, int NT, bool QLDS, bool SB, bool OA, int SPLIT, bool RM>
 __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_fwd_pipe_kernel(
     const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
     const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
   // dynamic LDS per wave: [Q fragments (QLDS)] [block list] [bitmap] [row masks]
   extern __shared__ __align__(16) unsigned char psm_all[];
   unsigned char* psm = psm_all + (threadIdx.x >> 6) *
-                                     pipe_wave_lds(D, NT, QLDS, k_slots, NB, rowmask != nullptr);
+                                     pipe_wave_lds(D, NT, QLDS, k_slots, NB, RM);
   constexpr int QBYTES = QLDS ? NT * KS * 64 * 16 : 0;
   int32_t* blist = reinterpret_cast<int32_t*>(psm + QBYTES);
 
@@ -213,9 +213,9 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
   const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   uint32_t* bits = reinterpret_cast<uint32_t*>(blist + k_slots);
   const int n_words = (min(t, NB - 1) >> 5) + 1;     // visible blocks are <= t
-  // per-row keep masks of the visited blocks (bit r: tile row r keeps the
-  // block), listed beside blist; without them every row attends every block
-  const uint64_t* rmk = rowmask != nullptr ? rowmask + idx_off : nullptr;
+  // RM: per-row keep masks of the visited blocks (bit r: tile row r keeps the
+  // block), listed beside blist; without RM every row attends every block
+  const uint64_t* rmk = RM ? rowmask + idx_off : nullptr;
   uint64_t* mlist = reinterpret_cast<uint64_t*>(
       blist + ((k_slots + (NB + 31) / 32 + 1) & ~1));
   for (int w = lane; w < n_words; w += 64) bits[w] = 0u;
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
     for (int j = 0; j < 4; ++j) {
       const int s = base0 + 64 * j + lane;
       blks[j] = s < k_slots ? idx[s] : -1;
-      mks[j] = rmk != nullptr && s < k_slots ? rmk[s] : 0ull;
+      mks[j] = RM && s < k_slots ? rmk[s] : 0ull;
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
       const uint64_t bal = __ballot(ok);
       if (ok) {
         blist[nv + __popcll(bal & lt_mask)] = blk;
-        if (rmk != nullptr) mlist[nv + __popcll(bal & lt_mask)] = mks[j];
+        if constexpr (RM) mlist[nv + __popcll(bal & lt_mask)] = mks[j];
         const uint32_t bit = 1u << (blk & 31);
         dup |= (atomicOr(&bits[blk >> 5], bit) & bit) != 0u;
       }
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
   wave_lds_sync();
   // with row masks the slots are visited in their order (the masks are
   // listed per slot); otherwise a list without repeats is re-sorted
-  if (rmk == nullptr && __ballot(dup) == 0) {
+  if (!RM && __ballot(dup) == 0) {
     int pos = 0;
     for (int w0 = 0; w0 < n_words; w0 += 64) {
       const int w = w0 + lane;
@@ -331,24 +331,35 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
   for (int nt = 0; nt < NT; ++nt) { m[nt] = -1e30f; l[nt] = 0.f; }
   bf16x8 pb[NT];
 
-  // Row-keep mask of half block u (wave-uniform), all rows without masks.
-  auto mbits = [&](int u) -> uint64_t {
-    if (rmk == nullptr) return ~0ull;
-    const uint64_t x = mlist[clamp_u(u) >> 1];
-    return (static_cast<uint64_t>(uni(static_cast<int>(x >> 32))) << 32) |
-           static_cast<uint32_t>(uni(static_cast<int>(x)));
+  // Row-keep mask of half block u as read from LDS (the reads are issued early
+  // and made wave-uniform where the mask is applied), all rows without RM.
+  auto mask_raw = [&](int u) -> uint2 {
+    if constexpr (RM) return *reinterpret_cast<const uint2*>(&mlist[clamp_u(u) >> 1]);
+    else return make_uint2(~0u, ~0u);
   };
   // Causal / bounds / row-keep mask (only half blocks crossing the diagonal
   // or N, or not kept by every row).
-  auto mask = [&](SBuf& st, int blk, int half, uint64_t mk) {
+  auto mask = [&](SBuf& st, int blk, int half, uint2 raw) {
     const int kbase = blk * kBlock + 32 * half;
+    // bit r of the word of row set nt: row 16 (nt & 1) + r of its 32 rows
+    uint32_t mw[2] = {~0u, ~0u};
+    if constexpr (RM) {
+      mw[0] = static_cast<uint32_t>(uni(static_cast<int>(raw.x)));
+      mw[1] = static_cast<uint32_t>(uni(static_cast<int>(raw.y)));
+    }
+    auto row_off = [&](int nt) -> bool {
+      if constexpr (!RM) return false;
+      const int set = rbase / 16 + nt;               // row set of the tile
+      const uint32_t word = set >= 2 ? mw[1] : mw[0];
+      return ((word >> (16 * (set & 1))) & (1u << r16)) == 0u;
+    };
     if (kbase + 31 <= row0 && kbase + 32 <= N) {
       // causally visible and in bounds: only rows without the keep bit
       // drop, each as a whole row set of S
-      if (mk != ~0ull) {
+      if (RM && (mw[0] & mw[1]) != ~0u) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-          const bool off = ((mk >> (rbase + 16 * nt + r16)) & 1ull) == 0;
+          const bool off = row_off(nt);
 #pragma unroll
           for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
@@ -360,7 +371,7 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const int row = row0 + 16 * nt + r16;
-        const bool off = ((mk >> (rbase + 16 * nt + r16)) & 1ull) == 0;
+        const bool off = row_off(nt);
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
@@ -655,6 +666,7 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
     // about 500 at head_dim 64, where the other wavefront covers the rest).
     auto step1 = [&](SBuf& cur, SBuf& nxt, int u) {
       const int rk = blk_raw(u + 2), rm1 = blk_raw(u + 1);
+      const uint2 mr = mask_raw(u + 1);
       asm volatile("" : "+v"(lane_b));
       phase1(cur, nxt, ka);
       load_k(uni(rk), clamp_u(u + 2) & 1, ka);
@@ -665,7 +677,7 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
         asm volatile("" : "+v"(pin), "+v"(l[nt]));
         pb[nt] = __builtin_bit_cast(bf16x8, pin);
       }
-      mask(nxt, uni(rm1), (u + 1) & 1, mbits(u + 1));
+      mask(nxt, uni(rm1), (u + 1) & 1, mr);
       if constexpr (OA) {
         float alpha[NT];
         const bool moved = phase2(nxt, va, alpha);
@@ -684,7 +696,7 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
       }
       qk(sa, ka);
       load_k(uni(blk_raw(1)), clamp_u(1) & 1, ka);
-      mask(sa, uni(blk_raw(0)), 0, mbits(0));
+      mask(sa, uni(blk_raw(0)), 0, mask_raw(0));
       if (rowmax(sa)) rescale();
 #pragma unroll
       for (int e = 0; e < E1ST; ++e) softmax_elem(sa, e);
@@ -705,6 +717,7 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
     // block ids of K(u+3), the mask of S(u+1) and V(u+2), read from LDS
     // before phase 1 so that their latency hides behind it
     const int rk = blk_raw(u + 3), rm1 = blk_raw(u + 1), rv = blk_raw(u + 2);
+    const uint2 mr = mask_raw(u + 1);
     phase1(cur, nxt, kc);
     commit(cur);
     gchar* kp = k_ptr(uni(rk), clamp_u(u + 3) & 1);
@@ -716,7 +729,7 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
       asm volatile("" : "+v"(pin), "+v"(l[nt]));
       pb[nt] = __builtin_bit_cast(bf16x8, pin);
     }
-    mask(nxt, uni(rm1), (u + 1) & 1, mbits(u + 1));
+    mask(nxt, uni(rm1), (u + 1) & 1, mr);
     // K(u+3) into kc (free once phase 1 has read K(u+1)): one slab every
     // second MFMA pair of phase 2 (the odd ones) rather than all eight at
     // once, so the four waves of a CU do not load in bursts (c2 / c3 / c4
@@ -754,7 +767,7 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
     qk(sa, ka);
     load_k(uni(blk_raw(2)), clamp_u(2) & 1, ka);
     load_v(uni(blk_raw(1)), 1, vb);
-    mask(sa, uni(blk_raw(0)), 0, mbits(0));
+    mask(sa, uni(blk_raw(0)), 0, mask_raw(0));
     if (rowmax(sa)) rescale();
 #pragma unroll
     for (int e = 0; e < E1ST; ++e) softmax_elem(sa, e);
@@ -886,7 +899,7 @@ constexpr int gen_waves() { return D > 128 ? 1 : 3; }
 // One launch (or the generations of one call): tile_order (optional) holds the
 // (b, t) tiles heaviest first (attn_tile_order) and enables the generations
 // above; without it, one launch with tiles by t descending.
-template <typename E, int D, int NT, bool QLDS, bool SB, bool OA, int SPLIT>
+template <typename E, int D, int NT, bool QLDS, bool SB, bool OA, int SPLIT, bool RM>
 static hipError_t launch_attn_pipe_t(const uint16_t* q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
                                      const uint16_t* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
                                      const uint16_t* vt, const int32_t* kv_idx,
@@ -900,10 +913,10 @@ static hipError_t launch_attn_pipe_t(const uint16_t* q, int64_t sq_b, int64_t sq
   const int units = B * Hk * Qt;
   constexpr int WPT = 4 / NT * SPLIT;
   size_t lds = static_cast<size_t>(WPT) *
-               pipe_wave_lds(D, NT, QLDS, k_slots, NB, rowmask != nullptr);
+               pipe_wave_lds(D, NT, QLDS, k_slots, NB, RM);
   if (lds < static_cast<size_t>(pipe_merge_lds(NT, SPLIT))) lds = pipe_merge_lds(NT, SPLIT);
   if (lds > 160 * 1024) return hipErrorInvalidConfiguration;
-  auto kern = attn_fwd_pipe_kernel<E, D, NT, QLDS, SB, OA, SPLIT>;
+  auto kern = attn_fwd_pipe_kernel<E, D, NT, QLDS, SB, OA, SPLIT, RM>;
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -941,15 +954,17 @@ static hipError_t launch_attn_pipe(const uint16_t* q, int64_t sq_b, int64_t sq_h
                                    int k_slots, float scale, uint16_t* out, int64_t so_b,
                                    int64_t so_h, int64_t so_m, hipStream_t stream,
                                    const int32_t* tile_order, int split) {
-#define UGBSA_PIPE(S_)                                                                          \
-  return launch_attn_pipe_t<E, D, NT, QLDS, SB, OA, S_>(                                       \
+#define UGBSA_PIPE(S_, RM_)                                                                     \
+  return launch_attn_pipe_t<E, D, NT, QLDS, SB, OA, S_, RM_>(                                  \
       q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx, rowmask, si_b, si_h, si_t, B, H, Hk, \
       M, N, Qt, k_slots, scale, out, so_b, so_h, so_m, stream, tile_order)
+#define UGBSA_PIPE_RM(S_) if (rowmask != nullptr) UGBSA_PIPE(S_, true); else UGBSA_PIPE(S_, false)
   if constexpr (!OA) {
-    if (split == 4) UGBSA_PIPE(4);
-    if (split == 2) UGBSA_PIPE(2);
+    if (split == 4) { UGBSA_PIPE_RM(4); }
+    if (split == 2) { UGBSA_PIPE_RM(2); }
   }
-  UGBSA_PIPE(1);
+  UGBSA_PIPE_RM(1);
+#undef UGBSA_PIPE_RM
 #undef UGBSA_PIPE
 }
 
