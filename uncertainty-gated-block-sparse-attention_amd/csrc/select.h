@@ -29,8 +29,8 @@
 // the CU, to the same buffer after a second barrier.  Each wave computes its 64 x CH score chunk on MFMA
 // (A = its Q tile, with the Quest sign split done once, from registers;
 // B = planes from LDS), max-pools it over rows in registers and appends CH
-// tile scores to its LDS row.  The row then goes through a 4-pass 8-bit radix
-// select for the k_slots-th best key, a ballot compaction of the winners
+// tile scores to its LDS row.  The row then goes through a search for the
+// k_slots-th best key (search_to_cand, select_to_cand), a ballot compaction of the winners
 // (ties at the cut taken in block order) and a register bitonic sort.
 //
 // Dump mode (ugbsa_score_dump, the diagnostic of src/dump_block_scores.py:
@@ -73,7 +73,7 @@ __host__ __device__ inline SelectLds select_lds(int P, int D, int NB, int KP, in
 }
 
 // Visible blocks whose keys the top-k keeps in registers (64 per lane step);
-// longer rows run the same radix select on their LDS row.
+// longer rows run a radix select on their LDS row.
 constexpr int kRegKeys = 32;
 
 // One radix-select step: hist holds 256 digit counts of the keys still in
@@ -147,6 +147,92 @@ __device__ inline uint32_t shrink_cand(uint64_t* cand, int n, int K, uint32_t* h
   }
   wave_lds_sync();
   return prefix;
+}
+
+// select_to_cand for rows of up to 512 blocks (K < n_vis <= 64 * RK): a threshold
+// search over register keys, about half the VALU work of the radix select and
+// no histogram round trips through LDS while a row is few registers.  Selection
+// launch with it and the sort sized to the winners: 40 heads x 16K tokens, 192
+// slots 102 -> 96 us; dump of 28 heads x 32K, 257 ranks 169 -> 163 us.  With 16
+// and 32 registers its counts cost what the radix passes do: 28 heads x 128K
+// 0.07 ms slower, so longer rows keep the radix select.
+template <int RK>
+__device__ __forceinline__ void search_to_cand(const float* trow, int n_vis, int K, uint64_t* cand,
+                                               int lane, uint64_t lt_mask) {
+  // The K-th largest key is built bit by bit: a candidate threshold is kept
+  // when at least K keys reach it (one compare per register, counted by the
+  // scalar unit), until exactly K do.  Unused slots hold key 0, below every
+  // score's; a test of the row length per slot would spill its conditions in
+  // the loop.  The search starts below the bits that every score except the
+  // two forced ones shares (their AND / OR over the wavefront).
+  uint32_t key[RK];
+  uint32_t kand = 0xFFFFFFFFu, kor = 0u;
+  static_for<RK>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    key[j] = 0u;
+    const int i = lane + 64 * j;
+    if (i < n_vis) {
+      key[j] = float_key(trow[i]);
+      if (i != 0 && i != n_vis - 1) { kand &= key[j]; kor |= key[j]; }
+    }
+  });
+  kand = wave_and_u32(kand, lane);
+  kor = wave_or_u32(kor, lane);
+  const uint32_t diff = kand ^ kor;
+  const int common = diff ? __clz(static_cast<int>(diff)) : 32;
+  const uint32_t cmask = common ? (0xFFFFFFFFu << (32 - common)) : 0u;
+  // the K-th key lies in the common prefix's range unless the two keys
+  // left out of it decide otherwise (only positions 0 and n_vis - 1,
+  // n_vis > K >= 1, can lie above or below it)
+  const uint32_t pre = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(kand & cmask)));
+  const uint32_t kf = float_key(trow[0]) & cmask, kl = float_key(trow[n_vis - 1]) & cmask;
+  const int above = __builtin_amdgcn_readfirstlane((kf > pre ? 1 : 0) + (kl > pre ? 1 : 0));
+  const int below = __builtin_amdgcn_readfirstlane((kf < pre ? 1 : 0) + (kl < pre ? 1 : 0));
+  uint32_t t = 0u;
+  int n_ge = 64 * RK, bit = 31;
+  if (K > above && K <= n_vis - below) {
+    t = pre;
+    n_ge = n_vis - below;
+    bit = __builtin_amdgcn_readfirstlane(31 - common);
+  }
+  for (; bit >= 0 && n_ge != K; --bit) {
+    const uint32_t c = t | (1u << bit);
+    int n = 0;
+    static_for<RK>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      n += __popcll(__ballot(key[j] >= c));
+    });
+    if (n >= K) {
+      t = c;
+      n_ge = n;
+    }
+  }
+  // exactly K keys reach t, or the first of those equal to it (in block
+  // order) complete the keys above it
+  int at = 0, need_eq = 0;
+  if (n_ge != K) {
+    int n_gt = 0;
+    static_for<RK>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      n_gt += __popcll(__ballot(key[j] > t));
+    });
+    need_eq = K - n_gt;
+  }
+  static_for<RK>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    bool take = key[j] >= t;
+    if (n_ge != K) {
+      const bool eq = key[j] == t;
+      const uint64_t be = __ballot(eq);
+      take = key[j] > t || (eq && static_cast<int>(__popcll(be & lt_mask)) < need_eq);
+      need_eq -= static_cast<int>(__popcll(be));   // below zero once none is left
+    }
+    const uint64_t bt = __ballot(take);
+    if (take)
+      cand[at + __popcll(bt & lt_mask)] =
+          (static_cast<uint64_t>(key[j]) << 32) | (0xFFFFFFFFu - static_cast<uint32_t>(lane + 64 * j));
+    at += __popcll(bt);
+  });
 }
 
 // Top-K of trow[0 .. n_vis) by (score desc, block asc) into cand[0 ..
@@ -294,21 +380,15 @@ __device__ __forceinline__ void select_to_cand(const float* trow, int n_vis, int
   }
 }
 
-// Loads cand[0 .. n_sel) into v (element e = lane + 64 r) and sorts it
-// descending: a register bitonic sort over KP elements.
-template <int KP>
-__device__ __forceinline__ void sort_cand(const uint64_t* cand, int n_sel, int lane,
-                                          uint64_t (&v)[KP / 64]) {
+// Sorts the first KP elements of v (element e = lane + 64 r) descending: a
+// register bitonic sort.
+template <int KP, int RT>
+__device__ __forceinline__ void bitonic_sort(uint64_t (&v)[RT], int lane) {
   constexpr int R = KP / 64;
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int e = lane + 64 * r;
-    v[r] = e < n_sel ? cand[e] : 0ull;
-  }
-  // bitonic sort, descending: stage (kk, j) compares element e with e ^ j,
-  // across registers for j >= 64, across lanes (register shuffles) below
+  // stage (kk, j) compares element e with e ^ j, across registers for j >= 64,
+  // across lanes (register shuffles) below
   constexpr int LOG_KP = KP == 64 ? 6 : KP == 128 ? 7 : KP == 256 ? 8 : 9;
-  static_assert((1 << LOG_KP) == KP, "KP is a power of two");
+  static_assert((1 << LOG_KP) == KP && R <= RT, "KP is a power of two within v");
   static_for<LOG_KP>([&](auto lk) {
     constexpr int kk = 2 << decltype(lk)::value;
     static_for<decltype(lk)::value + 1>([&](auto lj) {
@@ -329,6 +409,31 @@ __device__ __forceinline__ void sort_cand(const uint64_t* cand, int n_sel, int l
       for (int r = 0; r < R; ++r) v[r] = nv[r];
     });
   });
+}
+
+// Loads cand[0 .. n_sel) into v (element e = lane + 64 r) and sorts it
+// descending.  Tiles of fewer visible blocks than half the slots sort half as
+// many elements (and so on down to 64): a causal context of a few times k_slots
+// blocks has many.
+template <int KP>
+__device__ __forceinline__ void sort_cand(const uint64_t* cand, int n_sel, int lane,
+                                          uint64_t (&v)[KP / 64]) {
+  constexpr int R = KP / 64;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int e = lane + 64 * r;
+    v[r] = e < n_sel ? cand[e] : 0ull;
+  }
+  if constexpr (KP > 64) {
+    if (n_sel <= 64) return bitonic_sort<64>(v, lane);
+  }
+  if constexpr (KP > 128) {
+    if (n_sel <= 128) return bitonic_sort<128>(v, lane);
+  }
+  if constexpr (KP > 256) {
+    if (n_sel <= 256) return bitonic_sort<256>(v, lane);
+  }
+  bitonic_sort<KP>(v, lane);
 }
 
 // Score of rank e (0 = best) of a sorted v; -inf at ranks past n_sel.
@@ -667,11 +772,12 @@ __global__ __launch_bounds__(64 * kSelWaves) void select_kernel(
     wave_lds_sync();
     if (ts != nullptr)
       for (int i = lane; i < NB; i += 64) ts[i] = i < n_vis ? trow[i] : -INFINITY;
-    // register keys sized to the row (8, 16 or 32 per lane): the key loops
-    // are unrolled over the slots, so a short row runs far fewer of them
-    // (select at c2 0.175 -> 0.161 ms, c3 1.77 -> 1.72, c4 0.741 -> 0.705;
-    // 4 per lane for rows of up to 256 blocks gains nothing more)
-    if (n_vis <= 64 * 8) select_to_cand<8>(trow, n_vis, K, hist, cand, lane, lt_mask);
+    // register keys sized to the row (4, 8, 16 or 32 per lane): the key loops
+    // are unrolled over the slots, so a short row runs far fewer of them (with
+    // 8 / 16 / 32 against always 32: 28 heads x 32K 0.175 -> 0.161 ms, x 128K
+    // 1.77 -> 1.72 ms)
+    if (n_vis > K && n_vis <= 64 * 4) search_to_cand<4>(trow, n_vis, K, cand, lane, lt_mask);
+    else if (n_vis > K && n_vis <= 64 * 8) search_to_cand<8>(trow, n_vis, K, cand, lane, lt_mask);
     else if (n_vis <= 64 * 16) select_to_cand<16>(trow, n_vis, K, hist, cand, lane, lt_mask);
     else select_to_cand<kRegKeys>(trow, n_vis, K, hist, cand, lane, lt_mask);
   }
