@@ -26,7 +26,8 @@ def check(out, ref):
 # (H, M): 12 tiles and 72 (four wavefronts a tile), 360 (two), 720 (one); lists from none to every
 # visible block, so runs of no, one and several blocks, and one list in slot order (repeats)
 @pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float16),
-                                     (128, torch.bfloat16), (128, torch.float16)])
+                                     (128, torch.bfloat16), (128, torch.float16),
+                                     (256, torch.bfloat16), (256, torch.float16)])
 @pytest.mark.parametrize("H,M", [(4, 190), (4, 1150), (20, 1101), (40, 1150)])
 def test_tile_lists(hip_lib, D, dtype, H, M):
     print(f"[case] split lists D={D} {dtype} H={H} M={M}", flush=True)
@@ -53,7 +54,7 @@ def test_tile_lists(hip_lib, D, dtype, H, M):
                 assert (out[0, h, 64 * t:64 * t + 64] == 0).all()
 
 
-@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("H,M", [(4, 190), (20, 1101)])
 def test_row_masks(hip_lib, D, H, M):
     print(f"[case] split row masks D={D} H={H} M={M}", flush=True)
@@ -68,9 +69,10 @@ def test_row_masks(hip_lib, D, H, M):
     check(out, OA.keep_attention(f32np(q), f32np(k), f32np(v), keep.numpy(), D ** -0.5))
 
 
-def test_offsets_far_apart(hip_lib):
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_offsets_far_apart(hip_lib, D):
     """Runs whose row maxima differ by hundreds of log2 units merge without overflow."""
-    D, H, M = 128, 4, 1150
+    H, M = 4, 1150
     q, k, v = qkv(7, 1, H, H, M, D, torch.bfloat16)
     k[:, :, 640:704] *= 40.0
     nb = qt = (M + 63) // 64

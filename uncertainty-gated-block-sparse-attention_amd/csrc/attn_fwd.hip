@@ -252,16 +252,19 @@ static int pipe_slots(int D) { return D == 64 ? 2048 : 1024; }
 // a chain unsplit and 8 split (11-16 us against 1.8 us per block at head_dim
 // 128), so the rule compares (in blocks) the longest wavefront and the whole
 // work over the chip, plus a quarter of the longest for the ragged end, and
-// splits for at least 7 %.  Attention, us, 1 / 2 / 4 wavefronts (the rule's
+// splits for at least 7 % (25 % at head_dim 256, where a tile's runs in
+// different keys cost L2 hits: 16 heads, 32 blocks of 2K tokens 134 -> 79 us, 64
+// of 4K 232 -> 169, but 4 heads, 128 of 16K 460 -> 485).  Attention, us, 1 / 2 / 4 wavefronts (the rule's
 // choice first): head_dim 128, 28 heads, 8 blocks of 512 tokens 17.9 (4; 23.3,
 // 19.6), 16 of 1K 29.1 (2; 38.2, 40.5), 32 of 2K 63.6 (2; 69.0, 82.4), 64 of 4K
 // 138 (1; 152, 183); 8 heads, 32 of 2K 29.9 (4; 60.6, 40.4), 157 of 10K 230 (2;
 // 272, 240), 64 of 10K 144 (1; 155, 170); head_dim 64, 8 heads, 157 of 10K 147
 // (4; 249, 173), 16 heads, 32 of 8K 89 (1; 103, 103).
 static int attn_split(int64_t tiles, int Qt, int k_slots, int NB, int D, bool rowmask) {
-  if (NB > kGenBlocks || D > 128) return 1;
+  if (NB > kGenBlocks || (D > 128 && rowmask)) return 1;   // (attn_pipe.h: no such instance)
   const int64_t most = k_slots < Qt ? k_slots : Qt;             // longest list
   const double mean = most - 0.5 * most * (most - 1) / Qt;      // sum of min(t + 1, most) / Qt
+  const double gain = D > 128 ? 0.75 : 0.93;
   int best = 1;
   double best_t = 0.0;
   for (int s = 1; s <= 4; s *= 2) {
@@ -270,7 +273,7 @@ static int attn_split(int64_t tiles, int Qt, int k_slots, int NB, int D, bool ro
     const double longest = fixed + static_cast<double>(most) / s;
     const double all = tiles * (fixed * s + mean) / pipe_slots(D);
     const double t = (longest > all ? longest : all) + 0.25 * longest;
-    if (s == 1 || t < 0.93 * best_t) { best = s; best_t = t; }
+    if (s == 1 || t < gain * best_t) { best = s; best_t = t; }
   }
   return best;
 }
@@ -571,7 +574,7 @@ static hipError_t launch_attn_fwd_e(const uint16_t* q, int64_t sq_b, int64_t sq_
     if (D == 256)
       return launch_attn_pipe256(E::code, q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx, rowmask, si_b,
                                  si_h, si_t, B, H, Hk, M, N, Qt, k_slots, scale, out, so_b, so_h,
-                                 so_m, stream, tile_order);
+                                 so_m, stream, tile_order, split);
     if (D == 128)
       return launch_attn_pipe<E, 128, 4, false, false>(q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx,
                                           rowmask, si_b, si_h, si_t, B, H, Hk, M, N, Qt, k_slots,

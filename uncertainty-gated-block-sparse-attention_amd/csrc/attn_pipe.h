@@ -45,7 +45,7 @@ namespace ugbsa {
 // 199 / 360, two with the row sums 186 / 339 (816 TFLOP/s).
 // The tile's kv_idx row is compacted into LDS once (visited blocks only), so
 // sentinel and invisible slots cost nothing in the loop.
-// SPLIT > 1 (head_dim 64 / 128, calls of few tiles): the workgroup's SPLIT
+// SPLIT > 1 (calls of few tiles): the workgroup's SPLIT
 // wavefronts all hold the tile's rows, each visits one run of its list, and
 // they merge (O, m, l) through LDS.
 // Per-wave LDS bytes of attn_fwd_pipe_kernel: Q fragments (QLDS), block
@@ -69,8 +69,14 @@ __host__ __device__ constexpr int pipe_merge_lds(int NT, int split) {
   return split == 1 ? 0 : split * NT * 64 * (kMergeDt * 16 + 8);
 }
 
-template <typename E, int D, int NT, bool QLDS, bool SB, bool OA, int SPLIT, bool RM>
-__global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_fwd_pipe_kernel(
+// Template parameter CFG of the kernel: row sets per wavefront (NT), wavefronts
+// per tile (SPLIT) and row masks (RM); the plain tile kernel's is its NT.
+constexpr int pipe_cfg(int NT, int split, bool rm) { return NT + 16 * (split - 1) + (rm ? 256 : 0); }
+constexpr int cfg_nt(int cfg) { return cfg % 16; }
+constexpr int cfg_split(int cfg) { return cfg / 16 % 16 + 1; }
+
+template <typename E, int D, int CFG, bool QLDS, bool SB, bool OA>
+__global__ __launch_bounds__(64 * (4 / cfg_nt(CFG)) * cfg_split(CFG), D == 64 ? 2 : 1) void attn_fwd_pipe_kernel(
     const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
     const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
     const uint16_t* __restrict__ vt, const int32_t* __restrict__ kv_idx,
@@ -79,14 +85,17 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
     uint16_t* __restrict__ out, int64_t so_b, int64_t so_h, int64_t so_m,
     const int32_t* __restrict__ tile_order, int unit0, int unit_end, int grp) {
   constexpr int KS = D / 32, DT = D / 16, BM = 64;
+  constexpr int NT = cfg_nt(CFG), SPLIT = cfg_split(CFG);
+  constexpr bool RM = CFG >= 256;
   // NT = 4: one wavefront per 64-row tile; NT = 2: two wavefronts, 32 rows
   // each, which run independently (each keeps its own copy of the list)
   static_assert(NT == 4 || NT == 2, "a wavefront takes 64 or 32 rows of a tile");
   // OA: O^T accumulates in AGPRs (a 64-row tile at head_dim 256 fills all
   // 256 of them), written only by the P.V MFMAs of the SB loop
   static_assert(!OA || SB, "AGPR accumulators are used by the single-set loop");
-  // (at head_dim 256 the merge spilled 200-600 bytes of O^T per lane)
-  static_assert(SPLIT == 1 || (NT == 4 && !OA), "a split tile's wavefronts hold all of its rows");
+  // (at head_dim 256 the split row-masked forms would spill 132-160 bytes)
+  static_assert(SPLIT == 1 || (NT == 4 && !(OA && RM)),
+                "a split tile's wavefronts hold all of its rows");
   const int wave = SPLIT > 1 ? 0 : threadIdx.x >> 6;
   const int part_id = SPLIT > 1 ? threadIdx.x >> 6 : 0;
   // dynamic LDS per wave: [Q fragments (QLDS)] [block list] [bitmap] [row masks]
@@ -806,8 +815,13 @@ __global__ __launch_bounds__(64 * (4 / NT) * SPLIT, D == 64 ? 2 : 1) void attn_f
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int j = 0; j < kMergeDt; ++j)
+        for (int j = 0; j < kMergeDt; ++j) {
+          // with OA one fragment at a time leaves its AGPRs (read ahead of
+          // the barriers together they spilled 200-600 bytes)
+          if constexpr (OA) asm volatile("" : "+a"(o[ps * kMergeDt + j][nt]));
           mo[((part_id * NT + nt) * kMergeDt + j) * 64 + lane] = o[ps * kMergeDt + j][nt];
+          if constexpr (OA) __builtin_amdgcn_sched_barrier(0);
+        }
       __syncthreads();
 #pragma unroll
       for (int rs = 0; rs < RS; ++rs) {
@@ -916,7 +930,7 @@ static hipError_t launch_attn_pipe_t(const uint16_t* q, int64_t sq_b, int64_t sq
                pipe_wave_lds(D, NT, QLDS, k_slots, NB, RM);
   if (lds < static_cast<size_t>(pipe_merge_lds(NT, SPLIT))) lds = pipe_merge_lds(NT, SPLIT);
   if (lds > 160 * 1024) return hipErrorInvalidConfiguration;
-  auto kern = attn_fwd_pipe_kernel<E, D, NT, QLDS, SB, OA, SPLIT, RM>;
+  auto kern = attn_fwd_pipe_kernel<E, D, pipe_cfg(NT, SPLIT, RM), QLDS, SB, OA>;
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -959,7 +973,10 @@ static hipError_t launch_attn_pipe(const uint16_t* q, int64_t sq_b, int64_t sq_h
       q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx, rowmask, si_b, si_h, si_t, B, H, Hk, \
       M, N, Qt, k_slots, scale, out, so_b, so_h, so_m, stream, tile_order)
 #define UGBSA_PIPE_RM(S_) if (rowmask != nullptr) UGBSA_PIPE(S_, true); else UGBSA_PIPE(S_, false)
-  if constexpr (!OA) {
+  if constexpr (OA) {
+    if (split == 4 && rowmask == nullptr) UGBSA_PIPE(4, false);
+    if (split == 2 && rowmask == nullptr) UGBSA_PIPE(2, false);
+  } else {
     if (split == 4) { UGBSA_PIPE_RM(4); }
     if (split == 2) { UGBSA_PIPE_RM(2); }
   }

@@ -130,7 +130,7 @@ hipError_t launch_attn_pipe256(int elem, const uint16_t* q, int64_t sq_b, int64_
                                int64_t si_t, int B, int H, int Hk, int M, int N, int Qt,
                                int k_slots, float scale, uint16_t* out, int64_t so_b,
                                int64_t so_h, int64_t so_m, hipStream_t stream,
-                               const int32_t* tile_order);
+                               const int32_t* tile_order, int split);
 
 // _compute_kv_idx on the GPU: per (b, h, block_m-row tile) the blocks any row
 // of keep [B, H, M, NB] (uint8, contiguous) keeps, ascending, NB-padded to
