@@ -565,7 +565,11 @@ static hipError_t launch_attn_fwd_e(const uint16_t* q, int64_t sq_b, int64_t sq_
     const int64_t tiles = static_cast<int64_t>(B) * H * Qt;
     const int split = attn_split(tiles, Qt, k_slots, NBk, D, rowmask != nullptr);
     const int32_t* tile_order = nullptr;
-    if (order_ws != nullptr && tiles * split > pipe_slots(D)) {   // else all start at once
+    // Not ranked: calls whose wavefronts all start at once, and row-masked calls
+    // in one launch, whose lists are unions over 64 rows and so grow with t (the
+    // two ranking launches are 10 us of a 241 us layer of 28 heads x 4K).
+    if (order_ws != nullptr && tiles * split > pipe_slots(D) &&
+        (rowmask == nullptr || NBk > kGenBlocks)) {
       hipError_t e = launch_attn_tile_order(kv_idx, si_b, si_h, si_t, B, H, Qt, k_slots, NBk,
                                             order_ws, stream);
       if (e != hipSuccess) return e;
