@@ -232,6 +232,14 @@ int ugbsa_attn_prepare_kv(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_
                           int B, int Hk, int N, int D, int dtype, int block_m, void* workspace,
                           int64_t workspace_elems, void* stream);
 
+/* ugbsa_block_summary and ugbsa_attn_prepare_kv (block_m 64) in one launch that
+ * reads K once: what both write, bit for bit.  A ugbsa_attn_fwd with v NULL on
+ * the same workspace follows the selection. */
+int ugbsa_prepare_layer(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n, int64_t sk_d,
+                        const void* v, int64_t sv_b, int64_t sv_h, int64_t sv_n, int64_t sv_d,
+                        int B, int Hk, int N, int D, int dtype, int mode, void* planes,
+                        void* workspace, int64_t workspace_elems, void* stream);
+
 /* Kernel 3 — block-sparse causal attention over kv_idx.
  * Replaces block_sparse_attn_v2 (src/triton_block_attn.py:267-298) and its
  * kernel _fwd_kernel_v2 (:184-264).  q [B, H, M, D], k/v [B, Hk, N, D] in dtype

@@ -57,6 +57,8 @@ SIGNATURES = {
     "ugbsa_attn_workspace_elems": (_i64, [_i, _i, _i, _i]),
     "ugbsa_attn_prepare_kv": (_i, [_p, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64,
                                    _i, _i, _i, _i, _i, _i, _p, _i64, _p]),
+    "ugbsa_prepare_layer": (_i, [_p, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64,
+                                 _i, _i, _i, _i, _i, _i, _p, _p, _i64, _p]),
     "ugbsa_attn_fwd": (_i, [_p, _i64, _i64, _i64, _i64,
                             _p, _i64, _i64, _i64, _i64,
                             _p, _i64, _i64, _i64, _i64,

@@ -92,6 +92,21 @@ def block_sparse_attn_v2(q, k, v, kv_idx, scale, block_n=64, block_m=64,
     return out
 
 
+def attn_prepared(q, k, kv_idx, scale, out, workspace):
+    """``block_sparse_attn_v2`` (64-row tiles) on a workspace that already holds K and V in
+    operand order (``ugbsa_prepare_layer``); k only for its shape."""
+    q = _operand("q", q)
+    B, H, M, D = q.shape
+    Hk, N = k.shape[1], k.shape[2]
+    _capi.check(_capi.lib().ugbsa_attn_fwd(
+        q.data_ptr(), *q.stride(), k.data_ptr(), *k.stride(), None, 0, 0, 0, 1,
+        kv_idx.data_ptr(), *kv_idx.stride(),
+        B, H, Hk, M, N, D, _capi.dtype_code(q.dtype), kv_idx.shape[2], kv_idx.shape[3], 64,
+        float(scale), out.data_ptr(), *out.stride(), workspace.data_ptr(), workspace.numel(),
+        _capi.stream_ptr(q.device)), "block_sparse_attn_v2")
+    return out
+
+
 def _unwatched(q, k, v):
     """Whether a launch on the tensors' data pointers is all there is to a call: dense tensors,
     outside autograd, autocast, tracing, modes and functional transforms."""

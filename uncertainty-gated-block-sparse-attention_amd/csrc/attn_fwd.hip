@@ -40,6 +40,7 @@
 #include "common.h"
 #include "launch.h"
 #include "attn_pipe.h"
+#include "kv_operand.h"
 
 namespace ugbsa {
 
@@ -69,18 +70,13 @@ __global__ __launch_bounds__(256) void v_block_transpose_kernel(
   }
 }
 
-// K and V of one 64-key block in the pipelined kernel's operand order: for
-// each 32-key half block, K as 2 (mt) x KS 1 KiB slabs and V^T as DT 1 KiB
-// slabs, where lane L's 16 bytes sit at 16 * L of its slab.  K slab (mt, ks)
-// lane (g4, r16) = K[key 8 * (r16 >> 2) + 4 * mt + (r16 & 3)][32 * ks + 8 * g4 ..];
-// V^T slab dt lane (g4, r16) = V[keys 8 * g4 .. 8 * g4 + 7][16 * dt + r16].
-// Every operand load of the attention loop is then one contiguous KiB.
+// K and V of one 64-key block into the operand copies (kv_operand.h).
 template <int D>
 __global__ __launch_bounds__(256) void kv_operand_kernel(
     const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
     const uint16_t* __restrict__ v, int64_t sv_b, int64_t sv_h, int64_t sv_n, int Hk, int N,
     int NB, uint16_t* __restrict__ kop, uint16_t* __restrict__ vop) {
-  constexpr int KS = D / 32, DT = D / 16, CH = D / 8, ROW = D + 8;
+  constexpr int CH = D / 8, ROW = D + 8;
   // head_dim 256: K and V pass through one LDS tile in turn (two would
   // exceed 64 KiB of static LDS)
   constexpr bool ONE = D > 128;
@@ -106,29 +102,12 @@ __global__ __launch_bounds__(256) void kv_operand_kernel(
   };
   stage(true, !ONE);
   const int64_t base = ((static_cast<int64_t>(b) * Hk + h) * NB + blk) * kBlock * D;
-  // K: 2 halves x 2 mt x KS slabs x 64 lanes
-  for (int i = threadIdx.x; i < 2 * 2 * KS * 64; i += 256) {
-    const int lane = i & 63, slab = i >> 6;
-    const int ks = slab % KS, mt = (slab / KS) & 1, half = slab / (2 * KS);
-    const int g4 = lane >> 4, r16 = lane & 15;
-    const int key = 32 * half + 8 * (r16 >> 2) + 4 * mt + (r16 & 3);
-    *reinterpret_cast<u32x4*>(kop + base + static_cast<int64_t>(i) * 8) =
-        *reinterpret_cast<const u32x4*>(&kt[key][32 * ks + 8 * g4]);
-  }
+  write_k_slabs<D>(kt, kop + base);
   if (ONE) {
     __syncthreads();
     stage(false, true);
   }
-  // V^T: 2 halves x DT slabs x 64 lanes
-  for (int i = threadIdx.x; i < 2 * DT * 64; i += 256) {
-    const int lane = i & 63, slab = i >> 6;
-    const int dt = slab % DT, half = slab / DT;
-    const int g4 = lane >> 4, r16 = lane & 15;
-    i16x8 w;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) w[j] = static_cast<short>(vt_[32 * half + 8 * g4 + j][16 * dt + r16]);
-    *reinterpret_cast<i16x8*>(vop + base + static_cast<int64_t>(i) * 8) = w;
-  }
+  write_vt_slabs<D>(vt_, vop + base);
 }
 
 // Work of each (b, t) tile of 64 query rows: the visited slots of its

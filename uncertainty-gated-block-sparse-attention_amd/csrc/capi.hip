@@ -232,6 +232,32 @@ int ugbsa_attn_prepare_kv(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_
                     "attn_prepare_kv");
 }
 
+int ugbsa_prepare_layer(const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n, int64_t sk_d,
+                        const void* v, int64_t sv_b, int64_t sv_h, int64_t sv_n, int64_t sv_d,
+                        int B, int Hk, int N, int D, int dtype, int mode, void* planes,
+                        void* workspace, int64_t workspace_elems, void* stream) {
+  int rc = check_dims(B, Hk, Hk, D, dtype);
+  if (rc) return rc;
+  if ((rc = check_bf16_operand("k", k, sk_b, sk_h, sk_n, sk_d))) return rc;
+  if ((rc = check_bf16_operand("v", v, sv_b, sv_h, sv_n, sv_d))) return rc;
+  if (N < 1) return fail(UGBSA_EARG, "N must be positive");
+  if (mode != UGBSA_MODE_MEAN && mode != UGBSA_MODE_QUEST) return fail(UGBSA_EARG, "unknown score mode %d", mode);
+  if (planes == nullptr) return fail(UGBSA_EARG, "planes is null");
+  if (!aligned16(planes)) return fail(UGBSA_ELAYOUT, "planes must be 16-byte aligned");
+  if (workspace == nullptr || !aligned16(workspace)) return fail(UGBSA_EARG, "workspace must be a 16-byte aligned buffer");
+  if (workspace_elems < kv_copy_elems(B, Hk, N, D))
+    return fail(UGBSA_EARG, "workspace of %lld elements holds less than the K/V operand copies (%lld)",
+                (long long)workspace_elems, (long long)kv_copy_elems(B, Hk, N, D));
+  if (kv_copy_elems(1, 1, N, D) * 2 > 0xFFFFFFFFLL)
+    return fail(UGBSA_EARG, "one KV head's K/V copy exceeds 4 GiB (N=%d, D=%d)", N, D);
+  return hip_result(ugbsa::launch_summary_operand(
+                        static_cast<const uint16_t*>(k), sk_b, sk_h, sk_n,
+                        static_cast<const uint16_t*>(v), sv_b, sv_h, sv_n, B, Hk, N, D, dtype, mode,
+                        static_cast<uint16_t*>(planes), static_cast<uint16_t*>(workspace),
+                        static_cast<hipStream_t>(stream)),
+                    "prepare_layer");
+}
+
 }  // extern "C"
 
 namespace {

@@ -34,6 +34,12 @@ hipError_t launch_block_summary(const uint16_t* k, int64_t sk_b, int64_t sk_h, i
                                 uint16_t* planes, hipStream_t stream, uint16_t* pool = nullptr,
                                 int rep = 1);
 
+// launch_block_summary and launch_attn_prepare (64-row tiles) in one launch.
+hipError_t launch_summary_operand(const uint16_t* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
+                                  const uint16_t* v, int64_t sv_b, int64_t sv_h, int64_t sv_n,
+                                  int B, int Hk, int N, int D, int elem, int mode,
+                                  uint16_t* planes, uint16_t* ws, hipStream_t stream);
+
 // Extra modes of the selection kernel.
 //  dump != 0: per-tile order statistics of the unforced tile scores, ranked
 //             k_slots = rho_k + 1 deep, written instead of kv_idx;

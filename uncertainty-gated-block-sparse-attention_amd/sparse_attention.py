@@ -50,7 +50,8 @@ import torch
 import torch.nn.functional as F
 
 import _capi
-from block_attn import attn_workspace, block_sparse_attn, block_sparse_attn_v2, decode_attn
+from block_attn import (attn_prepared, attn_workspace, block_sparse_attn, block_sparse_attn_v2,
+                        decode_attn)
 
 BLOCK = 64   # tokens per selection block (src/sparse_attention.py:51)
 
@@ -169,8 +170,9 @@ class SelectionResult:
 
 
 def select_v2(query, key_states, scaling, block_m=64, sel: Selector = None,
-              want_tile_score=False) -> SelectionResult:
-    """Run kernels 1, 2 and the router; return kv_idx plus the router state."""
+              want_tile_score=False, planes=None) -> SelectionResult:
+    """Run kernels 1, 2 and the router; return kv_idx plus the router state.
+    ``planes``: kernel 1's output for ``key_states`` where the caller has it."""
     sel = SEL if sel is None else sel
     assert block_m == BLOCK, "selection tiles are 64 rows"
     assert query.shape[-2] == key_states.shape[-2], (
@@ -191,7 +193,8 @@ def select_v2(query, key_states, scaling, block_m=64, sel: Selector = None,
     k_base, k_slots = budgets(n_blocks, sel)
     mode = _capi.MODE_QUEST if use_quest(sel) else _capi.MODE_MEAN
 
-    planes = block_summary(key_states, mode)
+    if planes is None:
+        planes = block_summary(key_states, mode)
     is_router = sel.mode == "router" and k_base < k_slots
     kv_idx = torch.empty(B, H, q_tiles, k_slots, dtype=torch.int32, device=dev)
     sigma = torch.empty(B, H, q_tiles, dtype=torch.float32, device=dev) if is_router else None
@@ -272,7 +275,12 @@ def _block_select_kv_idx_v2(query, key_states, scaling, block_m=64):
     the repeat_kv'd [B, H, N, D] tensor (as the reference passes) or the GQA
     [B, Hk, N, D] one.
     """
-    res = select_v2(query, key_states, scaling, block_m)
+    return _select_logged(query, key_states, scaling, block_m)
+
+
+def _select_logged(query, key_states, scaling, block_m=64, planes=None):
+    """``select_v2``'s kv_idx with the ``SEL.log`` diagnostics (:726-746)."""
+    res = select_v2(query, key_states, scaling, block_m, planes=planes)
     kv_idx = res.kv_idx
     if SEL.log:
         if res.uncertain is not None:
@@ -286,6 +294,36 @@ def _block_select_kv_idx_v2(query, key_states, scaling, block_m=64):
         SEL.kept_blocks[layer_idx] = kept.cpu()
         SEL.budget_samples.append(float(res.k_slots))
     return kv_idx
+
+
+# The functions the dispatcher resolves at call time, as defined here: while
+# nothing wraps them, a layer prepares summaries and operand copies together.
+_SELECT_V2, _ATTN_V2 = _block_select_kv_idx_v2, block_sparse_attn_v2
+
+
+def _prepare_layer(query, key, value):
+    """(key, planes, workspace) of one sparse layer from one launch, or None where the
+    selector and the attention are to see the tensors themselves: the summary planes of
+    ``SEL``'s backbone and the attention workspace with K and V in operand order."""
+    if not (query.is_cuda and key.is_cuda and value.is_cuda and query.dim() == key.dim() == 4
+            and key.shape == value.shape and key.dtype == value.dtype == query.dtype
+            and key.device == value.device == query.device
+            and query.dtype in (torch.bfloat16, torch.float16)
+            and key.shape[0] == query.shape[0] and key.shape[3] == query.shape[3]
+            and query.shape[1] % key.shape[1] == 0 and query.shape[3] in (64, 128, 256)):
+        return None
+    key, value = _contig_rows(key), _contig_rows(value)
+    B, Hk, N, D = key.shape
+    lib = _capi.lib()
+    mode = _capi.MODE_QUEST if use_quest() else _capi.MODE_MEAN
+    planes = torch.empty(lib.ugbsa_summary_elems(B, Hk, N, D, mode), dtype=key.dtype,
+                         device=key.device)
+    ws = attn_workspace(B, Hk, N, D, key.device)
+    _capi.check(lib.ugbsa_prepare_layer(
+        key.data_ptr(), *key.stride(), value.data_ptr(), *value.stride(), B, Hk, N, D,
+        _capi.dtype_code(key.dtype), mode, planes.data_ptr(), ws.data_ptr(), ws.numel(),
+        _capi.stream_ptr(key.device)), "prepare layer")
+    return key, planes, ws
 
 
 @dataclass
@@ -507,14 +545,23 @@ def block_sparse_attention(module, query, key, value, attention_mask,
         f"sparse prefill needs query length == key length (got {Q} vs {key.shape[-2]})")
     if SEL.kernel_v2 and SEL.mode in ("topk", "router", "quest"):
         ev = PROF.start("v2_select") if is_prefill else None
-        kv_idx = _block_select_kv_idx_v2(query, key, scaling)   # resolved at call time
+        prep = (_prepare_layer(query, key, value) if _block_select_kv_idx_v2 is _SELECT_V2
+                and block_sparse_attn_v2 is _ATTN_V2 else None)
+        if prep is not None:
+            key, planes, ws = prep
+            kv_idx = _select_logged(query, key, scaling, planes=planes)
+        else:
+            kv_idx = _block_select_kv_idx_v2(query, key, scaling)   # resolved at call time
         PROF.stop(ev)
         ev = PROF.start("v2_kernel") if is_prefill else None
         B, _, S, D = query.shape
         out = torch.empty(B, S, H, D, dtype=query.dtype, device=query.device)
-        ws = attn_workspace(B, Hk, key.shape[-2], D, query.device)
-        block_sparse_attn_v2(query, key, value, kv_idx, scale=scaling, block_n=BLOCK,
-                             out=out.transpose(1, 2), workspace=ws)
+        if prep is not None:
+            attn_prepared(query, key, kv_idx, scaling, out.transpose(1, 2), ws)
+        else:
+            ws = attn_workspace(B, Hk, key.shape[-2], D, query.device)
+            block_sparse_attn_v2(query, key, value, kv_idx, scale=scaling, block_n=BLOCK,
+                                 out=out.transpose(1, 2), workspace=ws)
         PROF.stop(ev)
         return out, None
 
