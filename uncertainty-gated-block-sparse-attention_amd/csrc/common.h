@@ -333,6 +333,12 @@ __device__ __forceinline__ uint32_t wave_or_u32(uint32_t x, int lane) {
   return x | xor_lanes<1>(x, lane);
 }
 
+// Lanes below this one whose bit is set in a ballot.
+__device__ __forceinline__ int lanes_below(uint64_t ballot) {
+  return static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(ballot >> 32),
+                          __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ballot), 0u)));
+}
+
 // Exclusive prefix sum across the wavefront.
 __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t x, int lane) {
   uint32_t incl = x;

@@ -110,8 +110,7 @@ __device__ __forceinline__ int radix_digit(const uint32_t* hist, int lane, int& 
 // largest score key tau, then a stable compaction of the keys above tau and
 // the first (in cand order, i.e. lowest block) of those equal to it.
 // Returns tau; n must exceed K.
-__device__ inline uint32_t shrink_cand(uint64_t* cand, int n, int K, uint32_t* hist, int lane,
-                                       uint64_t lt_mask) {
+__device__ inline uint32_t shrink_cand(uint64_t* cand, int n, int K, uint32_t* hist, int lane) {
   uint32_t prefix = 0, pmask = 0;
   int remaining = K;
   for (int shift = 24; shift >= 0; shift -= 8) {
@@ -139,9 +138,9 @@ __device__ inline uint32_t shrink_cand(uint64_t* cand, int n, int K, uint32_t* h
     const bool gt = i < n && key > prefix;
     const bool eq = i < n && key == prefix;
     const uint64_t be = __ballot(eq);
-    const bool keep = gt || (eq && eq_seen + __popcll(be & lt_mask) < need_eq);
+    const bool keep = gt || (eq && eq_seen + lanes_below(be) < need_eq);
     const uint64_t bk = __ballot(keep);
-    if (keep) cand[out + __popcll(bk & lt_mask)] = x;
+    if (keep) cand[out + lanes_below(bk)] = x;
     out += __popcll(bk);
     eq_seen += __popcll(be);
   }
@@ -158,7 +157,7 @@ __device__ inline uint32_t shrink_cand(uint64_t* cand, int n, int K, uint32_t* h
 // 0.07 ms slower, so longer rows keep the radix select.
 template <int RK>
 __device__ __forceinline__ void search_to_cand(const float* trow, int n_vis, int K, uint64_t* cand,
-                                               int lane, uint64_t lt_mask) {
+                                               int lane) {
   // The K-th largest key is built bit by bit: a candidate threshold is kept
   // when at least K keys reach it (one compare per register, counted by the
   // scalar unit), until exactly K do.  Unused slots hold key 0, below every
@@ -224,12 +223,12 @@ __device__ __forceinline__ void search_to_cand(const float* trow, int n_vis, int
     if (n_ge != K) {
       const bool eq = key[j] == t;
       const uint64_t be = __ballot(eq);
-      take = key[j] > t || (eq && static_cast<int>(__popcll(be & lt_mask)) < need_eq);
+      take = key[j] > t || (eq && lanes_below(be) < need_eq);
       need_eq -= static_cast<int>(__popcll(be));   // below zero once none is left
     }
     const uint64_t bt = __ballot(take);
     if (take)
-      cand[at + __popcll(bt & lt_mask)] =
+      cand[at + lanes_below(bt)] =
           (static_cast<uint64_t>(key[j]) << 32) | (0xFFFFFFFFu - static_cast<uint32_t>(lane + 64 * j));
     at += __popcll(bt);
   });
@@ -240,7 +239,7 @@ __device__ __forceinline__ void search_to_cand(const float* trow, int n_vis, int
 // The wave's LDS row, histogram and candidate buffer; wave-local.
 template <int RK = kRegKeys>
 __device__ __forceinline__ void select_to_cand(const float* trow, int n_vis, int K, uint32_t* hist,
-                                               uint64_t* cand, int lane, uint64_t lt_mask) {
+                                               uint64_t* cand, int lane) {
   if (n_vis > K) {
     // Radix select of the K-th largest key tau (8-bit digits from the most
     // significant), then the keys > tau and the first (K - #greater) keys
@@ -319,11 +318,11 @@ __device__ __forceinline__ void select_to_cand(const float* trow, int n_vis, int
             const uint64_t bg = __ballot(gt), be = __ballot(eq);
             const uint64_t comp = (static_cast<uint64_t>(key[j]) << 32) | (0xFFFFFFFFu - static_cast<uint32_t>(i));
             if (gt) {
-              const int pos = cnt_gt + __popcll(bg & lt_mask);
+              const int pos = cnt_gt + lanes_below(bg);
               if (pos < n_gt) cand[pos] = comp;
             }
             if (eq) {
-              const int pos = cnt_eq + __popcll(be & lt_mask);
+              const int pos = cnt_eq + lanes_below(be);
               if (pos < need_eq) cand[n_gt + pos] = comp;
             }
             cnt_gt += __popcll(bg);
@@ -363,11 +362,11 @@ __device__ __forceinline__ void select_to_cand(const float* trow, int n_vis, int
       const uint64_t bg = __ballot(gt), be = __ballot(eq);
       const uint64_t comp = (static_cast<uint64_t>(key) << 32) | (0xFFFFFFFFu - static_cast<uint32_t>(i));
       if (gt) {
-        const int pos = cnt_gt + __popcll(bg & lt_mask);
+        const int pos = cnt_gt + lanes_below(bg);
         if (pos < n_gt) cand[pos] = comp;
       }
       if (eq) {
-        const int pos = cnt_eq + __popcll(be & lt_mask);
+        const int pos = cnt_eq + lanes_below(be);
         if (pos < need_eq) cand[n_gt + pos] = comp;
       }
       cnt_gt += __popcll(bg);
@@ -450,11 +449,19 @@ __device__ __forceinline__ float sorted_value(const uint64_t (&v)[R], int e, int
 // Blocks per LDS chunk: 32 while a block's planes are at most 512 bytes, else 16.
 __host__ __device__ constexpr int select_chunk(int P, int D) { return P * D <= 256 ? 32 : 16; }
 
+// Wavefronts per SIMD the kernel's registers leave room for: three at 168 or
+// fewer (K means at head_dim 128 take 165 once the pair's tile, head and row
+// length are scalars; selector of 40 heads x 16K tokens 114 us with two, 102
+// with three), two for the sign-split Quest tile and head_dim 256.
+__host__ __device__ constexpr int sel_eu_waves(int D, bool quest, bool rows) {
+  return !rows && (D == 64 || (D == 128 && !quest)) ? 3 : 2;
+}
+
 // W: pairs (waves) per workgroup; wpb: workgroups per (b, KV head); nbuf:
 // plane chunk buffers in LDS, 2 (double-buffered) or 1 (a second barrier
 // per chunk), as the launcher sized the workgroup's LDS.
 template <typename E, int D, bool QUEST, int KP, bool STREAM, bool ROWS>
-__global__ __launch_bounds__(64 * kSelWaves) void select_kernel(
+__global__ __launch_bounds__(64 * kSelWaves, sel_eu_waves(D, QUEST, ROWS)) void select_kernel(
     const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
     const uint16_t* __restrict__ planes, const float* __restrict__ bscale, int B, int Hk, int M,
     int N, int NB, int Qt, int grp,
@@ -482,7 +489,7 @@ __global__ __launch_bounds__(64 * kSelWaves) void select_kernel(
   const SelectLds L = select_lds(P, D, NB, KP, CH, STREAM);
 
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // the pair's values in SGPRs
   const int g4 = lane >> 4, r16 = lane & 15;
   const int nthreads = blockDim.x;
 
@@ -520,7 +527,6 @@ __global__ __launch_bounds__(64 * kSelWaves) void select_kernel(
   const int64_t row_id = (static_cast<int64_t>(b) * H + h) * Qt + t;
   float* ts = tile_score != nullptr ? tile_score + row_id * NB : nullptr;
   const int K = k_slots;
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   // streaming rows: candidates kept so far and the score key they all beat
   int cnt = 0;
   uint32_t cut = 0u;
@@ -727,12 +733,12 @@ __global__ __launch_bounds__(64 * kSelWaves) void select_kernel(
           const bool take = ok && (!have_cut || key > cut);
           const uint64_t bal = __ballot(take);
           if (take)
-            cand[cnt + __popcll(bal & lt_mask)] =
+            cand[cnt + lanes_below(bal)] =
                 (static_cast<uint64_t>(key) << 32) | (0xFFFFFFFFu - static_cast<uint32_t>(blk));
           cnt += __popcll(bal);
           if (cnt > stream_cap(KP) - CH) {
             wave_lds_sync();
-            cut = shrink_cand(cand, cnt, K, hist, lane, lt_mask);
+            cut = shrink_cand(cand, cnt, K, hist, lane);
             cnt = K;
             have_cut = true;
           }
@@ -763,7 +769,7 @@ __global__ __launch_bounds__(64 * kSelWaves) void select_kernel(
   if constexpr (STREAM) {
     if (ts != nullptr)
       for (int i = n_vis + lane; i < NB; i += 64) ts[i] = -INFINITY;
-    if (cnt > K) shrink_cand(cand, cnt, K, hist, lane, lt_mask);
+    if (cnt > K) shrink_cand(cand, cnt, K, hist, lane);
   } else {
     if (lane == 0 && !aux.dump) {
       trow[0] = kFMax;
@@ -776,10 +782,10 @@ __global__ __launch_bounds__(64 * kSelWaves) void select_kernel(
     // are unrolled over the slots, so a short row runs far fewer of them (with
     // 8 / 16 / 32 against always 32: 28 heads x 32K 0.175 -> 0.161 ms, x 128K
     // 1.77 -> 1.72 ms)
-    if (n_vis > K && n_vis <= 64 * 4) search_to_cand<4>(trow, n_vis, K, cand, lane, lt_mask);
-    else if (n_vis > K && n_vis <= 64 * 8) search_to_cand<8>(trow, n_vis, K, cand, lane, lt_mask);
-    else if (n_vis <= 64 * 16) select_to_cand<16>(trow, n_vis, K, hist, cand, lane, lt_mask);
-    else select_to_cand<kRegKeys>(trow, n_vis, K, hist, cand, lane, lt_mask);
+    if (n_vis > K && n_vis <= 64 * 4) search_to_cand<4>(trow, n_vis, K, cand, lane);
+    else if (n_vis > K && n_vis <= 64 * 8) search_to_cand<8>(trow, n_vis, K, cand, lane);
+    else if (n_vis <= 64 * 16) select_to_cand<16>(trow, n_vis, K, hist, cand, lane);
+    else select_to_cand<kRegKeys>(trow, n_vis, K, hist, cand, lane);
   }
   wave_lds_sync();
 
@@ -843,15 +849,18 @@ static hipError_t launch_select_t(const uint16_t* q, int64_t sq_b, int64_t sq_h,
   const SelectLds L = select_lds(2, D, NB, KP, select_chunk(2, D), STREAM);
   constexpr int kLdsMax = 160 * 1024;
   // W (tile, head) pairs per workgroup, one wavefront each: the W that
-  // keeps the most wavefronts on a CU, given its LDS and at most 8 resident
-  // waves (about 230 VGPRs each), counting 10 % more when two or more
-  // workgroups share the CU (one's top-k then overlaps another's scoring);
-  // ties go to the larger W, which stages each plane chunk for more pairs,
-  // and to two chunk buffers over one (one fewer barrier per chunk; one
-  // buffer wins where it alone fits a second workgroup, as at head_dim 256
-  // with three planes: 2.55 -> 2.33 ms at 128K keys).  W < 4 counts half:
-  // such workgroups cannot prefetch a whole chunk into registers (they are
-  // only chosen when a long key range leaves no room in LDS for more waves).
+  // keeps the most wavefronts on a CU, given its LDS and the resident waves
+  // its registers allow (8, or 12 in four-wave workgroups), counting 10 % more
+  // when two or more workgroups share the CU (one's top-k then overlaps
+  // another's scoring); ties go to the larger W, which stages each plane chunk
+  // for more pairs, and to two chunk buffers over one (one fewer barrier per
+  // chunk; one buffer wins where it alone fits another workgroup).  W < 4 counts
+  // half: such workgroups cannot prefetch a whole chunk into registers (they
+  // are only chosen when a long key range leaves no room in LDS for more
+  // waves).  Two workgroups of six waves were slower than two of four (1.31
+  // against 0.75 ms, K means at 40 heads x 64K), so with three waves per SIMD
+  // workgroups of more than four are left to rows that fill a CU's LDS alone.
+  constexpr int kEu = sel_eu_waves(D, QUEST, ROWS);
   int W = 0, nbuf = 2;
   double best = -1.0;
   for (int nb = 2; nb >= 1; --nb)
@@ -859,7 +868,8 @@ static hipError_t launch_select_t(const uint16_t* q, int64_t sq_b, int64_t sq_h,
       const size_t lds_w = nb * static_cast<size_t>(L.chunk_bytes) + static_cast<size_t>(w) * L.wave_bytes;
       if (lds_w > static_cast<size_t>(kLdsMax)) break;
       int per_cu = static_cast<int>(kLdsMax / lds_w);
-      if (per_cu > 8 / w) per_cu = 8 / w;
+      if (per_cu > 4 * kEu / w) per_cu = 4 * kEu / w;
+      if (kEu == 3 && w > 4 && static_cast<size_t>(kLdsMax) / lds_w > 1) continue;
       const double active = per_cu * static_cast<double>(w) * (per_cu >= 2 ? 1.1 : 1.0) *
                             (w < 4 ? 0.5 : 1.0);
       if (active > best || (active == best && nb == nbuf)) { best = active; W = w; nbuf = nb; }

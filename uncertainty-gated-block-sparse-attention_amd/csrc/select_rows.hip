@@ -109,9 +109,7 @@ __device__ __forceinline__ int belief_count(const RowsArgs& a, const float (&x)[
   for (int j = 0; j < RK; ++j) {
     const bool take = kc.n_ge == n_sel ? key[j] >= kc.t : key[j] > kc.t;
     const uint64_t bal = __ballot(take);
-    if (take) cand[at + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
-                            static_cast<uint32_t>(bal >> 32),
-                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bal), 0u)))] = key[j];
+    if (take) cand[at + lanes_below(bal)] = key[j];
     at += __popcll(bal);
   }
   for (int e = at + lane; e < n_sel; e += 64) cand[e] = kc.t;   // ties at the cut
