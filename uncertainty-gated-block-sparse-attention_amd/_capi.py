@@ -112,7 +112,8 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch._C._cuda_getCurrentRawStream(device.index)   # no Stream object per launch
+    index = torch.cuda.current_device() if device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(index)   # no Stream object per launch
 
 
 def ptr(t) -> int | None:

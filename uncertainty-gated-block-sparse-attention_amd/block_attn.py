@@ -114,7 +114,7 @@ def _unwatched(q, k, v):
     return not ((torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad))
                 or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
                 or torch.is_autocast_enabled("cuda") or torch.autograd.forward_ad._current_level >= 0
-                or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
+                or torch._C._get_tracing_state() is not None
                 or wrapped(q) or wrapped(k) or wrapped(v)
                 or q.is_nested or k.is_nested or v.is_nested
                 or not (q.layout is k.layout is v.layout is torch.strided))
@@ -128,6 +128,8 @@ def decode_attn(q, k, v, scale):
     bf16 / fp16 tensors of one device, head_dim 64, 128 or 256, in a layout read in place (unit
     head_dim stride, 16-byte aligned rows), with nothing watching the call.
     """
+    if torch.compiler.is_compiling():     # first: the compiler folds it and traces SDPA
+        return None
     if not (type(q) is type(k) is type(v) is torch.Tensor and q.is_cuda and k.is_cuda and v.is_cuda
             and isinstance(scale, float) and q.dim() == 4 and k.dim() == 4
             and (q.dtype is torch.bfloat16 or q.dtype is torch.float16)

@@ -280,7 +280,10 @@ def _block_select_kv_idx_v2(query, key_states, scaling, block_m=64):
 
 def _select_logged(query, key_states, scaling, block_m=64, planes=None):
     """``select_v2``'s kv_idx with the ``SEL.log`` diagnostics (:726-746)."""
-    res = select_v2(query, key_states, scaling, block_m, planes=planes)
+    if planes is None:
+        res = select_v2(query, key_states, scaling, block_m)
+    else:
+        res = select_v2(query, key_states, scaling, block_m, planes=planes)
     kv_idx = res.kv_idx
     if SEL.log:
         if res.uncertain is not None:
@@ -298,7 +301,7 @@ def _select_logged(query, key_states, scaling, block_m=64, planes=None):
 
 # The functions the dispatcher resolves at call time, as defined here: while
 # nothing wraps them, a layer prepares summaries and operand copies together.
-_SELECT_V2, _ATTN_V2 = _block_select_kv_idx_v2, block_sparse_attn_v2
+_AS_DEFINED = (_block_select_kv_idx_v2, select_v2, block_summary, block_sparse_attn_v2)
 
 
 def _prepare_layer(query, key, value):
@@ -545,8 +548,9 @@ def block_sparse_attention(module, query, key, value, attention_mask,
         f"sparse prefill needs query length == key length (got {Q} vs {key.shape[-2]})")
     if SEL.kernel_v2 and SEL.mode in ("topk", "router", "quest"):
         ev = PROF.start("v2_select") if is_prefill else None
-        prep = (_prepare_layer(query, key, value) if _block_select_kv_idx_v2 is _SELECT_V2
-                and block_sparse_attn_v2 is _ATTN_V2 else None)
+        prep = None
+        if (_block_select_kv_idx_v2, select_v2, block_summary, block_sparse_attn_v2) == _AS_DEFINED:
+            prep = _prepare_layer(query, key, value)
         if prep is not None:
             key, planes, ws = prep
             kv_idx = _select_logged(query, key, scaling, planes=planes)
