@@ -12,12 +12,14 @@
 // times in the flattened tensor, so its k_quant-th smallest is the
 // ((k_quant - 1) / H + 1)-th smallest per-tile mean.
 //
-// The threshold needs every tile's sigma, so it runs as one 1024-thread
-// workgroup (an 8-bit radix select, 4 passes), followed by a grid-wide fill.
-// With row grain the per-tile head means stay in LDS while B * Qt <=
-// kRouterLdsMeans (every BASELINE shape, 1M tokens included), so the radix
-// passes and the decisions read LDS rather than L2; larger inputs and cell
-// grain select over sigma_eff in global memory.
+// The threshold needs every tile's sigma.  Up to kRouterOneLaunch values to
+// rank (per-tile means or cells) and kRouterOneLaunchCells cells, one launch
+// does everything: each workgroup ranks all values again, in registers, and
+// writes its own rows.  Above that the threshold comes from one 1024-thread
+// workgroup, followed by a grid-wide fill.  There, with row grain, the
+// per-tile head means stay in LDS while B * Qt <= kRouterLdsMeans (1M tokens
+// included), so the radix passes and the decisions read LDS rather than L2;
+// larger inputs and cell grain select over sigma_eff in global memory.
 #include "common.h"
 #include "launch.h"
 
@@ -43,13 +45,44 @@ __device__ __forceinline__ float head_sum_in_order(const float* __restrict__ x, 
 
 constexpr int kRouterLdsMeans = 16384;   // per-tile means held in LDS (64 KiB)
 
+constexpr int kRouterWaves = 16;   // 1024-thread workgroups
+
+// k-th smallest (1-based) key of a workgroup whose wavefronts each hold all
+// of them, KN a lane (absent ones 0xFFFFFFFF): the largest c with fewer than
+// kth keys below it, four bits a pass from the top.  Wavefront w counts the
+// keys below the pass's w-th candidate with ballots, so a pass is KN compares
+// and one barrier, with no histogram to clear, fold and scan and no atomics
+// that serialise on the digits the keys share.  Its work grows with KN: at
+// 4096 keys (KN = 64) it took 19.8 us against the radix select's 11.7, so
+// longer inputs keep the radix.
+template <int KN>
+__device__ __forceinline__ uint32_t block_kth_in_regs(const uint32_t (&key)[KN], uint32_t kth,
+                                                      uint32_t (*cnt)[kRouterWaves]) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t prefix = 0;
+  for (int shift = 28; shift >= 0; shift -= 4) {
+    const uint32_t c = prefix | (wave << shift);
+    uint32_t below = 0;
+#pragma unroll
+    for (int j = 0; j < KN; ++j) below += static_cast<uint32_t>(__popcll(__ballot(key[j] < c)));
+    uint32_t* row = cnt[(shift >> 2) & 1];   // two rows: one barrier a pass
+    if (lane == 0) row[wave] = below;
+    __syncthreads();
+    // candidate 0 is the prefix itself, below which there are fewer than kth
+    const bool ok = lane < kRouterWaves && row[lane & (kRouterWaves - 1)] < kth;
+    const uint32_t d = static_cast<uint32_t>(__popcll(__ballot(ok))) - 1u;
+    prefix |= d << shift;
+  }
+  return prefix;
+}
+
 // k-th smallest (1-based) of value_at(0 .. n - 1) by one workgroup: a
 // 4-pass 8-bit radix select over the order-preserving float keys (NaN above
 // every number); returns the key to every thread.  Each wavefront counts
 // into its own 256-bin histogram (hist holds kRouterWaves of them): the keys
 // of one pass mostly share their top digits, and one shared histogram would
 // serialise the LDS atomics of the whole workgroup on a few bins.
-constexpr int kRouterWaves = 16;   // 1024-thread workgroups
 template <class F>
 __device__ uint32_t block_kth_smallest(F value_at, int64_t n, int64_t kth, uint32_t* hist,
                                        uint32_t* s_prefix, uint32_t* s_remaining) {
@@ -177,11 +210,88 @@ __global__ __launch_bounds__(256) void router_fill_kernel(
   if (!uncertain[row]) kv_idx[row * k_slots + k_base + j] = NB;
 }
 
+// The whole pass in one launch for up to 64 KN values to rank: each workgroup
+// forms every value (per-tile head means or the cells) and ranks them for
+// itself, then decides and fills 64 rows at a time.  sigma_eff must not
+// overlap sigma, which other workgroups may still read.
+// Latency-bound: a chain of loads, 8 rank passes and the fill.  Against the
+// threshold and fill launches: 40 heads x 256 tiles 10.0 us (13.9 + 4.9),
+// 28 x 512 9.5 (14.5 + 5.0), 28 x 2048 23.0 (25.8 + 13.1).  The limits are
+// the registers of 2048 keys and the sigma every workgroup reads again.
+constexpr int kRouterOneLaunch = 2048;          // values: 32 registers a lane
+constexpr int64_t kRouterOneLaunchCells = 65536;  // 256 KiB read per workgroup
+template <int KN>
+__global__ __launch_bounds__(1024) void router_one_launch_kernel(
+    const float* __restrict__ sigma, int B, int H, int Qt, int grain, int rmode, float tau,
+    uint32_t kth, int32_t* __restrict__ kv_idx, int k_base, int k_slots, int NB,
+    float* __restrict__ sigma_eff, uint8_t* __restrict__ uncertain,
+    float* __restrict__ threshold) {
+  __shared__ float vals[64 * KN];
+  __shared__ uint32_t cnt[2][kRouterWaves];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rows = B * H * Qt;
+  const int n = grain == kGrainRow ? B * Qt : rows;   // <= 64 KN
+  for (int i = tid; i < n; i += 1024) {
+    if (grain == kGrainRow) {
+      const int b = i / Qt, t = i - b * Qt;
+      vals[i] = head_sum_in_order<32>(sigma + static_cast<int64_t>(b) * H * Qt + t, H, Qt) /
+                static_cast<float>(H);
+    } else {
+      vals[i] = sigma[i];
+    }
+  }
+  __syncthreads();
+  float thr = tau;
+  if (rmode == kRouterQuantile) {
+    uint32_t key[KN];
+#pragma unroll
+    for (int j = 0; j < KN; ++j)
+      key[j] = 64 * j + lane < n ? float_key(vals[64 * j + lane]) : 0xFFFFFFFFu;
+    thr = key_float(block_kth_in_regs<KN>(key, kth, cnt));
+  }
+  if (blockIdx.x == 0 && tid == 0 && threshold != nullptr) *threshold = thr;
+  for (int r0 = 64 * blockIdx.x; r0 < rows; r0 += 64 * gridDim.x) {
+    const int r = r0 + lane;
+    bool certain = false;
+    if (r < rows) {
+      const int bh = r / Qt;
+      const float e = vals[grain == kGrainRow ? (bh / H) * Qt + (r - bh * Qt) : r];
+      const bool unc = rmode == kRouterQuantile ? (e <= thr) : (e < tau);   // NaN: false
+      certain = !unc;
+      if (wave == 0) {
+        sigma_eff[r] = e;
+        uncertain[r] = unc;
+      }
+    }
+    const uint64_t fill = __ballot(certain);
+    for (int j = wave; j < 64; j += kRouterWaves) {
+      if ((fill >> j & 1) == 0) continue;
+      int32_t* extra = kv_idx + static_cast<int64_t>(r0 + j) * k_slots;
+      for (int x = k_base + lane; x < k_slots; x += 64) extra[x] = NB;
+    }
+  }
+}
+
 hipError_t launch_router(const float* sigma, int B, int H, int Qt, int grain, int rmode,
                          float tau, int64_t k_quant, int32_t* kv_idx, int k_base, int k_slots,
                          int NB, float* sigma_eff, uint8_t* uncertain, float* threshold,
                          hipStream_t stream) {
   const int64_t n_tiles = static_cast<int64_t>(B) * Qt;
+  const int64_t cells = n_tiles * H;
+  const int64_t n_rank = grain == kGrainRow ? n_tiles : cells;
+  const bool apart = sigma_eff + cells <= sigma || sigma + cells <= sigma_eff;
+  if (n_rank <= kRouterOneLaunch && cells <= kRouterOneLaunchCells && apart) {
+    const uint32_t kth = static_cast<uint32_t>(grain == kGrainRow ? (k_quant - 1) / H + 1
+                                                                  : k_quant);
+    const int64_t groups = (cells + 63) / 64;
+    const unsigned grid = static_cast<unsigned>(groups < 256 ? groups : 256);
+    auto* kernel = n_rank <= 512 ? router_one_launch_kernel<8>
+                                 : router_one_launch_kernel<32>;
+    kernel<<<grid, 1024, 0, stream>>>(sigma, B, H, Qt, grain, rmode, tau, kth, kv_idx, k_base,
+                                      k_slots, NB, sigma_eff, uncertain, threshold);
+    return hipGetLastError();
+  }
   const size_t lds = grain == kGrainRow && n_tiles <= kRouterLdsMeans
                          ? static_cast<size_t>(n_tiles) * sizeof(float) : 0;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(router_threshold_kernel),
@@ -284,6 +394,25 @@ __global__ __launch_bounds__(256) void router_rows_fill_kernel(
   }
   const bool wide = (NB & 7) == 0 && (reinterpret_cast<uintptr_t>(keep) & 7) == 0;
   uint64_t pending = __ballot(unc);
+  const int words = NB >> 3;   // 8-byte words a row
+  if (wide && words < __popcll(pending) * ((NB + 511) / 512)) {
+    // many short rows: all 64 as one run of words, a lane a word, the ones of
+    // untriggered cells left alone; taken where it needs fewer wavefront
+    // stores than row by row (28 heads x 4096 rows x 64 blocks, a quarter of
+    // the cells triggered: 13.7 -> 6.0 us)
+    const uint32_t row0 = static_cast<uint32_t>(c0 % M);
+    for (int x = lane; x < 64 * words; x += 64) {
+      const int j = x / words;
+      if ((pending >> j & 1) == 0) continue;
+      const int b0 = 8 * (x - j * words);
+      const int last = static_cast<int>((row0 + j) % static_cast<uint32_t>(M)) / kBlock;
+      uint64_t w = 0;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) w |= static_cast<uint64_t>(b0 + q <= last) << (8 * q);
+      *reinterpret_cast<uint64_t*>(keep + (c0 + j) * NB + b0) = w;
+    }
+    return;
+  }
   while (pending) {
     const int j = __ffsll(static_cast<long long>(pending)) - 1;
     pending &= pending - 1;
