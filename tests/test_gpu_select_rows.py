@@ -39,6 +39,21 @@ def test_keep_and_margin(hip_lib, nb, mode, kw):
     check(mode, kw, q, k)
 
 
+# a mass that is never reached: every row keeps the k_max best ranks, rows of fewer visible blocks
+# than that too (their total is 1 within 1e-6, so no row sits near either top_p)
+@pytest.mark.parametrize("nb,k_max", [(66, 66), (157, 112), (157, 64), (300, 200)])
+@pytest.mark.parametrize("top_p", [1.00002, 1.5])
+def test_belief_mass_never_reached(hip_lib, nb, k_max, top_p):
+    print(f"[case] belief nb={nb} k_max={k_max} top_p={top_p}", flush=True)
+    g = torch.Generator().manual_seed(nb)
+    q = torch.randn(1, 2, 64 * nb, 64, generator=g).to(torch.bfloat16)
+    k = (0.2 * torch.randn(1, 1, 64 * nb, 64, generator=g)).to(torch.bfloat16)
+    sel = make_sel(mode="belief", top_p=top_p, k_min=1, k_max=k_max)
+    res = sa.select_mask_v1(q.to(DEV), k.to(DEV), 0.125, sel=sel, want_scores=True)
+    check_on_kernel_scores(res, sel, 64 * nb)
+    assert res.keep[0, 0, 0].sum() == k_max        # one visible block, the rest lowest first
+
+
 @pytest.mark.parametrize("nb", [40, 100, 300])
 @pytest.mark.parametrize("mode,kw", [("topk", dict(budget_blocks=16)),
                                      ("router", dict(budget_blocks=24))])

@@ -143,6 +143,8 @@ __device__ __forceinline__ int belief_count(const RowsArgs& a, const float (&x)[
     carry = __shfl(c, 63, 64);
     cnt += __popcll(__ballot(e < a.K && c < a.top_p));
   }
+  // ranks past the sorted keys (none visible) add no mass: all of them count, or none
+  if (a.K > KP && carry < a.top_p) cnt += a.K - KP;
   int count = cnt + 1;
   if (count < a.k_min) count = a.k_min;
   if (count > a.k_max) count = a.k_max;
@@ -207,7 +209,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs& a, int64_t bh, int row
       int count = a.k_bud;
       KeyCut cut{1u, n_vis};               // every visible block
       if constexpr (BELIEF) {
-        // (RK 1: at most 64 visible blocks, so 64 sorted keys)
+        // (RK 1: at most 64 visible blocks, so 64 sorted keys, whatever K is)
         count = belief_count<RK, RK == 1 ? 64 : KP>(a, x, key, n_vis, cand, lane, cut.t);
         if (count < n_vis) {
           cut.n_ge = 0;
