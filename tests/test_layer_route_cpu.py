@@ -1,0 +1,78 @@
+"""Which entry points a sparse layer calls, with what, without a GPU: host tensors that pass for
+device ones, and a library that records its calls and launches nothing."""
+
+import pytest
+import torch
+
+import _capi
+import sparse_attention as sa
+
+LAUNCHES = {name for name, (res, args) in _capi.SIGNATURES.items()
+            if res is _capi._i and args}              # the rest are host-side queries
+
+
+class Dev(torch.Tensor):
+    is_cuda = True
+
+
+class Recorder:
+    """The library with its launches recorded as (name, arguments); ``on[name]`` runs with each and
+    may return the call's status."""
+
+    def __init__(self, real):
+        self.real, self.calls, self.on = real, [], {}
+
+    def __getattr__(self, name):
+        if name not in LAUNCHES:
+            return getattr(self.real, name)
+
+        def launch(*args):
+            self.calls.append((name, args))
+            return self.on.get(name, lambda *a: 0)(*args) or 0
+        return launch
+
+    def names(self):
+        return [name for name, _ in self.calls]
+
+    def args(self, name):
+        found = [args for n, args in self.calls if n == name]
+        assert len(found) == 1, (name, self.names())
+        return found[0]
+
+
+@pytest.fixture
+def rec(monkeypatch):
+    rec = Recorder(_capi.lib())
+    monkeypatch.setattr(_capi, "lib", lambda: rec)
+    monkeypatch.setattr(_capi, "stream_ptr", lambda device: 0)
+    monkeypatch.setattr(sa, "SEL", sa.Selector())
+    sa.SEL.mode, sa.SEL.kernel_v2, sa.SEL.budget_blocks = "router", True, 8
+    sa.SEL.k_min = 2
+    return rec
+
+
+def qkv(B=1, H=4, Hk=2, S=2048, D=64):
+    return tuple(torch.zeros(B, h, S, D, dtype=torch.bfloat16).as_subclass(Dev)
+                 for h in (H, Hk, Hk))
+
+
+@pytest.mark.parametrize("before,after", [("quest", "mean"), ("mean", "quest")])
+def test_policy_changed_between_preparation_and_selection(rec, before, after):
+    """The planes are read as what they were made as, whatever SEL has become since."""
+    sa.SEL.router_score = before
+    rec.on["ugbsa_prepare_layer"] = lambda *a: setattr(sa.SEL, "router_score", after)
+    sa.block_sparse_attention(None, *qkv(), None, 0.125)
+    made, read = rec.args("ugbsa_prepare_layer"), rec.args("ugbsa_select")
+    assert made[15:17] == (read[13], made[16]) and read[5] == made[16]
+    assert read[13] == (_capi.MODE_QUEST if before == "quest" else _capi.MODE_MEAN)
+
+
+def test_planes_of_another_mode_are_refused(rec):
+    q, k, _ = qkv()
+    sa.SEL.router_score = "mean"
+    planes = sa.block_summary(k, _capi.MODE_QUEST)
+    with pytest.raises(AssertionError):
+        sa.select_v2(q, k, 0.125, planes=planes)
+    assert "ugbsa_select" not in rec.names()
+    sa.select_v2(q, k, 0.125, planes=planes, mode=_capi.MODE_QUEST)
+    assert rec.args("ugbsa_select")[13] == _capi.MODE_QUEST

@@ -170,9 +170,10 @@ class SelectionResult:
 
 
 def select_v2(query, key_states, scaling, block_m=64, sel: Selector = None,
-              want_tile_score=False, planes=None) -> SelectionResult:
+              want_tile_score=False, planes=None, mode=None) -> SelectionResult:
     """Run kernels 1, 2 and the router; return kv_idx plus the router state.
-    ``planes``: kernel 1's output for ``key_states`` where the caller has it."""
+    ``planes``: kernel 1's output for ``key_states`` where the caller has it, and
+    ``mode`` (``_capi.MODE_*``) the backbone it was made for (default: ``sel``'s)."""
     sel = SEL if sel is None else sel
     assert block_m == BLOCK, "selection tiles are 64 rows"
     assert query.shape[-2] == key_states.shape[-2], (
@@ -191,10 +192,15 @@ def select_v2(query, key_states, scaling, block_m=64, sel: Selector = None,
     n_blocks = (N + BLOCK - 1) // BLOCK
     q_tiles = (M + block_m - 1) // block_m
     k_base, k_slots = budgets(n_blocks, sel)
-    mode = _capi.MODE_QUEST if use_quest(sel) else _capi.MODE_MEAN
+    if mode is None:
+        mode = _capi.MODE_QUEST if use_quest(sel) else _capi.MODE_MEAN
 
     if planes is None:
         planes = block_summary(key_states, mode)
+    else:   # ugbsa_summary_elems of the mode: the selection reads all of them
+        per_block = 2 * D if mode == _capi.MODE_QUEST else 2 * D + 2
+        assert planes.numel() == B * Hk * n_blocks * per_block, (
+            "planes are not a block summary of key_states in this mode")
     is_router = sel.mode == "router" and k_base < k_slots
     kv_idx = torch.empty(B, H, q_tiles, k_slots, dtype=torch.int32, device=dev)
     sigma = torch.empty(B, H, q_tiles, dtype=torch.float32, device=dev) if is_router else None
@@ -278,12 +284,12 @@ def _block_select_kv_idx_v2(query, key_states, scaling, block_m=64):
     return _select_logged(query, key_states, scaling, block_m)
 
 
-def _select_logged(query, key_states, scaling, block_m=64, planes=None):
+def _select_logged(query, key_states, scaling, block_m=64, planes=None, mode=None):
     """``select_v2``'s kv_idx with the ``SEL.log`` diagnostics (:726-746)."""
     if planes is None:
         res = select_v2(query, key_states, scaling, block_m)
     else:
-        res = select_v2(query, key_states, scaling, block_m, planes=planes)
+        res = select_v2(query, key_states, scaling, block_m, planes=planes, mode=mode)
     kv_idx = res.kv_idx
     if SEL.log:
         if res.uncertain is not None:
@@ -305,9 +311,10 @@ _AS_DEFINED = (_block_select_kv_idx_v2, select_v2, block_summary, block_sparse_a
 
 
 def _prepare_layer(query, key, value):
-    """(key, planes, workspace) of one sparse layer from one launch, or None where the
+    """(key, planes, mode, workspace) of one sparse layer from one launch, or None where the
     selector and the attention are to see the tensors themselves: the summary planes of
-    ``SEL``'s backbone and the attention workspace with K and V in operand order."""
+    ``SEL``'s backbone, which backbone that is (``SEL`` may change before the selection), and
+    the attention workspace with K and V in operand order."""
     if not (query.is_cuda and key.is_cuda and value.is_cuda and query.dim() == key.dim() == 4
             and key.shape == value.shape and key.dtype == value.dtype == query.dtype
             and key.device == value.device == query.device
@@ -326,7 +333,7 @@ def _prepare_layer(query, key, value):
         key.data_ptr(), *key.stride(), value.data_ptr(), *value.stride(), B, Hk, N, D,
         _capi.dtype_code(key.dtype), mode, planes.data_ptr(), ws.data_ptr(), ws.numel(),
         _capi.stream_ptr(key.device)), "prepare layer")
-    return key, planes, ws
+    return key, planes, mode, ws
 
 
 @dataclass
@@ -552,8 +559,8 @@ def block_sparse_attention(module, query, key, value, attention_mask,
         if (_block_select_kv_idx_v2, select_v2, block_summary, block_sparse_attn_v2) == _AS_DEFINED:
             prep = _prepare_layer(query, key, value)
         if prep is not None:
-            key, planes, ws = prep
-            kv_idx = _select_logged(query, key, scaling, planes=planes)
+            key, planes, mode, ws = prep
+            kv_idx = _select_logged(query, key, scaling, planes=planes, mode=mode)
         else:
             kv_idx = _block_select_kv_idx_v2(query, key, scaling)   # resolved at call time
         PROF.stop(ev)
