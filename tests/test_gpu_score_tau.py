@@ -38,3 +38,20 @@ def test_tau_splits(hip_lib, S, D, mode, score, dtype):
     again = dbs.record(q.to(DEV), k.to(DEV), D ** -0.5, sel=sel)
     for name in ("g", "r", "sigma", "g_rho", "valid", "tau_hat"):
         assert np.array_equal(shard[name], again[name], equal_nan=True), name
+
+
+@pytest.mark.parametrize("mode,score,size", [("quest", "quest", 3e17), ("topk", "mean", 3e18),
+                                             ("quest", "quest", 1e-15), ("topk", "mean", 1e-15)])
+def test_tau_of_large_and_small_scores(hip_lib, mode, score, size):
+    """Squares whose sum over a workgroup leaves fp32's range while their mean does not."""
+    print(f"[case] tau of scores {size} {mode}", flush=True)
+    g = torch.Generator().manual_seed(5)
+    q = torch.randn(1, 4, 1025, 64, generator=g).to(torch.bfloat16)
+    k = (size * torch.randn(1, 2, 1025, 64, generator=g)).to(torch.bfloat16)
+    sel = sa.Selector()
+    sel.mode, sel.router_score, sel.budget_blocks = mode, score, 1
+    ref = OD.tau_hat(f32np(q), f32np(k), 0.5, sa.use_quest(sel))
+    if size > 1:                                     # 256 pairs x 17 blocks: one workgroup's sum
+        assert (256 * 17 * 2 * ref.astype(np.float64) ** 2 > 4 * float(np.finfo(np.float32).max)).all()
+    shard = dbs.record(q.to(DEV), k.to(DEV), 0.5, sel=sel)
+    np.testing.assert_allclose(shard["tau_hat"], ref, rtol=1e-4)

@@ -22,9 +22,9 @@
 // idle, 233 us; split over the chip with every wavefront reading the planes
 // from L2 (64-byte pieces of 16 rows an instruction) 41 us; through LDS 25 us
 // (0.6 PFLOP/s, launch ramp included).  Squares are summed per lane in fp64,
-// then over lanes and waves; the workgroup's sum goes to two fp32 halves (48
-// bits) in part_hi / part_lo, which score_tau_reduce_kernel adds in a fixed
-// order, so the result is deterministic.
+// then over lanes and waves; the workgroup's fp64 sum goes whole, as its upper
+// and lower 32 bits, to part_hi / part_lo, and score_tau_reduce_kernel adds the
+// sums in a fixed order, so the result is deterministic.
 #include "common.h"
 #include "launch.h"
 
@@ -42,7 +42,7 @@ __global__ __launch_bounds__(64 * kTauWaves) void score_tau_kernel(
     const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
     const uint16_t* __restrict__ planes, const float* __restrict__ bscale, int Hk, int M, int NB,
     int grp, int n_pairs, int stride, float scaling, int nb_range, int64_t part_stride,
-    float* __restrict__ part_hi, float* __restrict__ part_lo) {
+    uint32_t* __restrict__ part_hi, uint32_t* __restrict__ part_lo) {
   constexpr int KS = D / 32;
   constexpr int P = 2;
   constexpr int QSETS = QUEST ? 2 : 1;
@@ -153,23 +153,23 @@ __global__ __launch_bounds__(64 * kTauWaves) void score_tau_kernel(
   if (threadIdx.x == 0) {
     double tot = 0.0;
     for (int w = 0; w < kTauWaves; ++w) tot += part[w];
-    const float hi = static_cast<float>(tot);
+    const uint64_t bits = __builtin_bit_cast(uint64_t, tot);
     const int64_t at = bh * part_stride + blockIdx.z * gridDim.y + blockIdx.y;
-    part_hi[at] = hi;
-    part_lo[at] = __builtin_isfinite(hi) ? static_cast<float>(tot - static_cast<double>(hi)) : 0.f;
+    part_hi[at] = static_cast<uint32_t>(bits >> 32);
+    part_lo[at] = static_cast<uint32_t>(bits);
   }
 }
 
 // tau_hat of one (b, h) from its workgroups' sums, added in their order.
 __global__ __launch_bounds__(64) void score_tau_reduce_kernel(
-    const float* __restrict__ part_hi, const float* __restrict__ part_lo, int64_t part_stride,
-    int parts, int n_pairs, int NB, float* __restrict__ tau_hat) {
+    const uint32_t* __restrict__ part_hi, const uint32_t* __restrict__ part_lo,
+    int64_t part_stride, int parts, int n_pairs, int NB, float* __restrict__ tau_hat) {
   if (threadIdx.x != 0) return;
   double tot = 0.0;
   const int64_t at = blockIdx.x * part_stride;
 #pragma unroll 8
   for (int i = 0; i < parts; ++i)
-    tot += static_cast<double>(part_hi[at + i]) + static_cast<double>(part_lo[at + i]);
+    tot += __builtin_bit_cast(double, static_cast<uint64_t>(part_hi[at + i]) << 32 | part_lo[at + i]);
   float tau = 0.f;
   if (n_pairs > 0) {
     const float mean = static_cast<float>(tot / (static_cast<double>(n_pairs) * NB));
@@ -194,6 +194,8 @@ static hipError_t launch_tau_t(const uint16_t* q, int64_t sq_b, int64_t sq_h, in
   // place among the (b, h)'s Qt scratch values: groups <= Qt, as a pass of
   // 8 MT >= 16 pairs spans at least 16 of the M - 1 rows.
   const int Qt = (M + kBlock - 1) / kBlock;
+  uint32_t* part_hi = reinterpret_cast<uint32_t*>(scratch_a);
+  uint32_t* part_lo = reinterpret_cast<uint32_t*>(scratch_b);
   const int groups = n_pairs > 0 ? ((n_pairs + 8 * MT - 1) / (8 * MT) + kTauWaves - 1) / kTauWaves : 0;
   int ranges = 1;
   if (groups > 0) {
@@ -208,12 +210,12 @@ static hipError_t launch_tau_t(const uint16_t* q, int64_t sq_b, int64_t sq_h, in
     score_tau_kernel<E, D, QUEST, MT><<<dim3(static_cast<unsigned>(B * H), groups, ranges),
                                         64 * kTauWaves, 0, stream>>>(
         q, sq_b, sq_h, sq_m, planes, QUEST ? nullptr : mean_descale(planes, B, Hk, NB, D), Hk, M,
-        NB, H / Hk, n_pairs, stride, scaling, tau_chunk(D) * per, Qt, scratch_a, scratch_b);
+        NB, H / Hk, n_pairs, stride, scaling, tau_chunk(D) * per, Qt, part_hi, part_lo);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   score_tau_reduce_kernel<<<dim3(static_cast<unsigned>(B * H)), 64, 0, stream>>>(
-      scratch_a, scratch_b, Qt, groups * ranges, n_pairs, NB, tau_hat);
+      part_hi, part_lo, Qt, groups * ranges, n_pairs, NB, tau_hat);
   return hipGetLastError();
 }
 
