@@ -116,3 +116,16 @@ def test_select_no_scratch_and_no_packed_fp32(asm, inst):
     assert len(entries) == 1
     m = re.search(r"\.private_segment_fixed_size:\s+(\d+)", entries[0])
     assert m and int(m.group(1)) == 0
+
+
+def test_no_instance_takes_scratch(asm):
+    """Every bf16 instance, the ones for rows of more than 4096 blocks (STREAM) and the row scores
+    among them: head_dim 64 / 128 / 256, both backbones, four slot counts streamed or not, and rows."""
+    meta = asm[asm.index(".amdgpu_metadata"):]
+    scratch = {}
+    for e in re.split(r"\n  - \.", meta):
+        name = re.search(r"\.name:\s+(_ZN5ugbsa13select_kernel\w+)", e)
+        if name:
+            scratch[name[1]] = int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", e)[1])
+    assert len(scratch) == 3 * 2 * (4 * 2 + 1)
+    assert {n: b for n, b in scratch.items() if b} == {}

@@ -452,16 +452,20 @@ __host__ __device__ constexpr int select_chunk(int P, int D) { return P * D <= 2
 // Wavefronts per SIMD the kernel's registers leave room for: three at 168 or
 // fewer (K means at head_dim 128 take 165 once the pair's tile, head and row
 // length are scalars; selector of 40 heads x 16K tokens 114 us with two, 102
-// with three), two for the sign-split Quest tile and head_dim 256.
-__host__ __device__ constexpr int sel_eu_waves(int D, bool quest, bool rows) {
-  return !rows && (D == 64 || (D == 128 && !quest)) ? 3 : 2;
+// with three), two for the sign-split Quest tile, head_dim 256, and K means at
+// head_dim 128 in streamed rows, which take 181: held to 168 they spill 8-9
+// registers into the chunk loop (8 heads x 512K tokens, 96 slots: 7.62 ms with
+// three, 6.80-6.88 with two; 268K tokens, 48 slots: 2.12 and 1.87).  Streamed
+// rows at head_dim 64 fit three (512K tokens, 96 slots: 4.79 ms with two, 3.76-3.88).
+__host__ __device__ constexpr int sel_eu_waves(int D, bool quest, bool stream, bool rows) {
+  return !rows && (D == 64 || (D == 128 && !quest && !stream)) ? 3 : 2;
 }
 
 // W: pairs (waves) per workgroup; wpb: workgroups per (b, KV head); nbuf:
 // plane chunk buffers in LDS, 2 (double-buffered) or 1 (a second barrier
 // per chunk), as the launcher sized the workgroup's LDS.
 template <typename E, int D, bool QUEST, int KP, bool STREAM, bool ROWS>
-__global__ __launch_bounds__(64 * kSelWaves, sel_eu_waves(D, QUEST, ROWS)) void select_kernel(
+__global__ __launch_bounds__(64 * kSelWaves, sel_eu_waves(D, QUEST, STREAM, ROWS)) void select_kernel(
     const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
     const uint16_t* __restrict__ planes, const float* __restrict__ bscale, int B, int Hk, int M,
     int N, int NB, int Qt, int grp,
@@ -860,7 +864,7 @@ static hipError_t launch_select_t(const uint16_t* q, int64_t sq_b, int64_t sq_h,
   // waves).  Two workgroups of six waves were slower than two of four (1.31
   // against 0.75 ms, K means at 40 heads x 64K), so with three waves per SIMD
   // workgroups of more than four are left to rows that fill a CU's LDS alone.
-  constexpr int kEu = sel_eu_waves(D, QUEST, ROWS);
+  constexpr int kEu = sel_eu_waves(D, QUEST, STREAM, ROWS);
   int W = 0, nbuf = 2;
   double best = -1.0;
   for (int nb = 2; nb >= 1; --nb)
