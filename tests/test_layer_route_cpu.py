@@ -76,3 +76,39 @@ def test_planes_of_another_mode_are_refused(rec):
     assert "ugbsa_select" not in rec.names()
     sa.select_v2(q, k, 0.125, planes=planes, mode=_capi.MODE_QUEST)
     assert rec.args("ugbsa_select")[13] == _capi.MODE_QUEST
+
+
+class Buckets:
+    """A profiler that notes its buckets among the recorded calls."""
+    enabled = True
+
+    def __init__(self, rec):
+        self.rec = rec
+
+    def start(self, name):
+        self.rec.calls.append((name, ()))
+        return name
+
+    def stop(self, name):
+        self.rec.calls.append(("end " + name, ()))
+
+
+@pytest.mark.parametrize("wrapped", [False, True])
+def test_profiler_buckets(rec, monkeypatch, wrapped):
+    """v2_select holds the selector and v2_kernel all of the attention, the K/V operand copies
+    included, whether or not a harness wraps the selector."""
+    monkeypatch.setattr(sa, "PROF", Buckets(rec))
+    if wrapped:
+        inner = sa._block_select_kv_idx_v2
+        monkeypatch.setattr(sa, "_block_select_kv_idx_v2", lambda *a, **kw: inner(*a, **kw))
+    q, k, v = qkv()
+    sa.block_sparse_attention(None, q, k, v, None, 0.125)
+    assert rec.names() == ["v2_select", "ugbsa_block_summary", "ugbsa_select", "ugbsa_router",
+                           "end v2_select", "v2_kernel", "ugbsa_attn_fwd", "end v2_kernel"]
+    assert rec.args("ugbsa_attn_fwd")[10] == v.data_ptr()      # not prepared: copied in this call
+
+
+def test_layer_without_profiler_prepares_in_one_launch(rec):
+    sa.block_sparse_attention(None, *qkv(), None, 0.125)
+    assert rec.names() == ["ugbsa_prepare_layer", "ugbsa_select", "ugbsa_router", "ugbsa_attn_fwd"]
+    assert rec.args("ugbsa_attn_fwd")[10] is None
