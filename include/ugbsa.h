@@ -210,6 +210,10 @@ int ugbsa_attn_fwd_rows(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
                         void* out, int64_t so_b, int64_t so_h, int64_t so_m, int64_t so_d,
                         void* workspace, int64_t workspace_elems, void* stream);
 
+/* LDS bytes that one wavefront of the 64-row-tile attention takes for Q, the
+ * list of a tile of k_slots slots and (row_masks != 0) its masks. */
+int64_t ugbsa_attn_wave_lds(int N, int D, int k_slots, int row_masks);
+
 /* Number of 16-bit elements of the attention workspace, in two parts:
  *   1. the K and V operand copies written by ugbsa_attn_prepare_kv,
  *      2 * B * Hk * NB * 64 * D elements (NB = ceil(N / 64));

@@ -1,11 +1,14 @@
 """Which entry points a sparse layer calls, with what, without a GPU: host tensors that pass for
 device ones, and a library that records its calls and launches nothing."""
 
+import ctypes
+
 import pytest
 import torch
 
 import _capi
 import sparse_attention as sa
+from block_attn import block_sparse_attn
 
 LAUNCHES = {name for name, (res, args) in _capi.SIGNATURES.items()
             if res is _capi._i and args}              # the rest are host-side queries
@@ -112,3 +115,21 @@ def test_layer_without_profiler_prepares_in_one_launch(rec):
     sa.block_sparse_attention(None, *qkv(), None, 0.125)
     assert rec.names() == ["ugbsa_prepare_layer", "ugbsa_select", "ugbsa_router", "ugbsa_attn_fwd"]
     assert rec.args("ugbsa_attn_fwd")[10] is None
+
+
+# a list with masks beside Q's fragments fills an eighth (head_dim 64) or a quarter of a CU's LDS
+@pytest.mark.parametrize("D,widest", [(64, 1013), (128, 1024), (256, 675)])
+def test_row_lists_as_wide_as_the_mask_keep_the_wavefronts(rec, D, widest):
+    waves = 8 if D == 64 else 4
+    for nb in (widest, widest + 1):
+        S = 64 * nb
+        q, k, v = qkv(1, 1, 1, S, D)
+        keep = torch.zeros(1, 1, S, nb, dtype=torch.bool).as_subclass(Dev)
+        rec.calls.clear()
+        rec.on["ugbsa_keep_kv_idx"] = lambda *a: ctypes.memset(a[8], 0, 4 * nb) and 0
+        block_sparse_attn(q, k, v, keep, 0.125)
+        slots = rec.args("ugbsa_attn_fwd_rows")[29]
+        assert slots == (nb if nb == widest else 1)       # past it: the longest list (none here)
+        listed = (nb + (nb + 31) // 32 + 1) // 2 * 2 * 4 + 8 * nb
+        fits = waves * ((listed + (0 if D == 128 else 128 * D)) + 15 & ~15) <= 160 * 1024
+        assert fits == (nb == widest) or D == 128         # (there 1024 is a cap on the copy to LDS)

@@ -189,11 +189,19 @@ def keep_kv_idx(keep, block_m=64, want_rowmask=True):
 
 
 # The row-masked attention takes the lists NB wide, without asking the device for
-# the longest one (40 us of host time a call), while a 64-row tile's list and
-# masks, 12 bytes a slot in LDS, leave every CU its eight wavefronts at head_dim
-# 64 (four at 128 and 256); the 32-row tile kernel walks every slot, so there
-# the longest list is worth a synchronisation.
+# the longest one (40 us of host time a call), up to 1024 blocks and while a 64-row
+# tile's list and masks, 12 bytes a slot in LDS beside Q's fragments, leave every CU
+# its wavefronts: eight at head_dim 64 (up to 1013 blocks), four at 128 (beyond 1024)
+# and 256 (up to 675; 8 heads x 768 blocks, at most 393 a tile: 7.56 ms with lists of
+# 768 slots, three wavefronts a CU, 6.17 with 393).  The 32-row tile kernel walks
+# every slot, so there the longest list is worth a synchronisation.
 _ROWS_LIST_BLOCKS = 1024
+_CU_LDS = 160 * 1024
+
+
+def _list_as_wide_as_mask(N, D, NB, block_m):
+    return (block_m == 64 and NB <= _ROWS_LIST_BLOCKS
+            and (8 if D == 64 else 4) * _capi.lib().ugbsa_attn_wave_lds(N, D, NB, 1) <= _CU_LDS)
 
 
 def block_sparse_attn(q, k, v, keep, scale, block_n=64, block_m=64,
@@ -215,7 +223,7 @@ def block_sparse_attn(q, k, v, keep, scale, block_n=64, block_m=64,
     Hk, N = k.shape[1], k.shape[2]
     assert H % Hk == 0, "query heads must be a multiple of KV heads"
     assert tuple(keep.shape[:3]) == (B, H, M), "keep [B, H, M, NB] expected"
-    if block_m == 64 and keep.shape[3] <= _ROWS_LIST_BLOCKS:
+    if _list_as_wide_as_mask(N, D, keep.shape[3], block_m):
         kv, rm, _ = _keep_lists(keep, block_m, True)
         max_kept = keep.shape[3]
     else:

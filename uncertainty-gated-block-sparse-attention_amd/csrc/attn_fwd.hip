@@ -220,6 +220,10 @@ static bool uses_pipe(int D, int block_m) {
 // Longest kv_idx row the pipelined kernel compacts into LDS.
 constexpr int kPipeMaxSlots = 16384;
 
+int attn_wave_lds(int N, int D, int k_slots, bool row_masks) {
+  return pipe_wave_lds(D, 4, D != 128, k_slots, (N + kBlock - 1) / kBlock, row_masks);
+}
+
 // Wavefronts of the pipelined kernel the chip holds at once: one per SIMD of
 // 256 CUs, two at head_dim 64.
 static int pipe_slots(int D) { return D == 64 ? 2048 : 1024; }

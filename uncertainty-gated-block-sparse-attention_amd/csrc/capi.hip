@@ -459,6 +459,10 @@ int ugbsa_keep_kv_idx(const uint8_t* keep, int B, int H, int M, int NB, int bloc
                     "keep_kv_idx");
 }
 
+int64_t ugbsa_attn_wave_lds(int N, int D, int k_slots, int row_masks) {
+  return ugbsa::attn_wave_lds(N, D, k_slots, row_masks != 0);
+}
+
 int64_t ugbsa_select_mask_workspace_elems(int B, int H, int M, int N) {
   const int64_t nb = (N + ugbsa::kBlock - 1) / ugbsa::kBlock;
   const int64_t mp = (M + ugbsa::kBlock - 1) / ugbsa::kBlock * ugbsa::kBlock;

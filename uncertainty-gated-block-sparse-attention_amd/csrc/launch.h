@@ -119,6 +119,9 @@ hipError_t launch_attn_fwd(const uint16_t* q, int64_t sq_b, int64_t sq_h, int64_
                            hipStream_t stream, const uint64_t* rowmask = nullptr,
                            int32_t* order_ws = nullptr);
 
+// LDS bytes of one wavefront of the 64-row-tile kernels.
+int attn_wave_lds(int N, int D, int k_slots, bool row_masks);
+
 // The (b, t) tiles of a kv_idx [B, H, Qt, k_slots] ordered by their visited
 // slots over all query heads, heaviest first (64-row tiles): ws holds 2 * B *
 // Qt int32 — the per-tile work, then the order (b * Qt + t per entry).
