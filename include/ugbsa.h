@@ -266,6 +266,9 @@ int ugbsa_attn_fwd(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m, int6
                    int64_t so_h, int64_t so_m, int64_t so_d, void* workspace,
                    int64_t workspace_elems, void* stream);
 
+/* Decode calls of fewer keys take no workspace. */
+#define UGBSA_DECODE_ONE_SPLIT 512
+
 /* fp32 elements of a ugbsa_decode workspace (0: none is needed). */
 int64_t ugbsa_decode_workspace_elems(int B, int H, int Hk, int N, int D);
 

@@ -158,3 +158,13 @@ def test_argument_errors_are_reported_without_launch(lib):
     rc = lib.ugbsa_score_dump(16, 0, 0, 8, 1, 16, 1, 8, 2, 256, 256, 128, _capi.DTYPE_BF16,
                               _capi.MODE_QUEST, 0.1, 2, 4, 16, 16, 16, 16, 16, 16, None, None)
     assert rc == -1 and b"rho_k" in lib.ugbsa_last_error()
+
+
+def test_decode_calls_without_a_workspace(lib):
+    # the binding asks for no workspace below the header's length, and none is needed there
+    text = open(HEADER).read()
+    line = int(re.search(r"#define UGBSA_DECODE_ONE_SPLIT\s+(\d+)", text)[1])
+    assert _capi.DECODE_ONE_SPLIT == line
+    for B, H, Hk, D in ((1, 1, 1, 64), (1, 28, 4, 128), (3, 64, 1, 256), (64, 64, 64, 128)):
+        assert all(lib.ugbsa_decode_workspace_elems(B, H, Hk, n, D) == 0 for n in range(1, line))
+    assert lib.ugbsa_decode_workspace_elems(1, 28, 4, line, 128) > 0

@@ -26,6 +26,7 @@ MODE_MEAN, MODE_QUEST = 0, 1
 GRAIN_CELL, GRAIN_ROW = 0, 1
 ROUTER_ABS, ROUTER_QUANTILE = 0, 1
 V1_TOPK, V1_BELIEF = 0, 1
+DECODE_ONE_SPLIT = 512
 
 # Every symbol include/ugbsa.h declares, with its ctypes signature.
 _i, _i64, _f, _p = ctypes.c_int, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p

@@ -151,7 +151,7 @@ def decode_attn(q, k, v, scale):
         return None
     lib = _capi.lib()
     out = torch.empty((B, 1, H, D), dtype=q.dtype, device=device)
-    n = lib.ugbsa_decode_workspace_elems(B, H, Hk, N, D) if N >= 512 else 0   # one split below
+    n = lib.ugbsa_decode_workspace_elems(B, H, Hk, N, D) if N >= _capi.DECODE_ONE_SPLIT else 0
     ws = torch.empty(n, dtype=torch.float32, device=device) if n else None
     _capi.check(lib.ugbsa_decode(
         pq, *sq, pk, *sk, pv, *sv, B, H, Hk, N, D, _capi.dtype_code(q.dtype), scale,

@@ -25,6 +25,7 @@
 // 1151 us at 32K.
 #include "common.h"
 #include "launch.h"
+#include "../../include/ugbsa.h"
 
 namespace ugbsa {
 
@@ -268,11 +269,10 @@ __global__ __launch_bounds__(kDecCombineThreads) void decode_combine_kernel(
 // against 7.7): the second launch costs less than a longer chain of steps.
 // At 512 keys the two are level (7.2 / 7.9 us on the GPU), and below, one split
 // spares the caller a workspace and a launch (10 against 14 us of host time).
-constexpr int kDecOneSplit = 512;
 int decode_splits(int B, int H, int Hk, int N, int D) {
   const int64_t units = static_cast<int64_t>(B) * Hk * ((H / Hk + dec_heads(D) - 1) / dec_heads(D));
   int64_t want = (D > 128 ? 256 : 512) / units;
-  const int64_t most = N < kDecOneSplit ? 1 : N / (kDecWaves * kDecStep);
+  const int64_t most = N < UGBSA_DECODE_ONE_SPLIT ? 1 : N / (kDecWaves * kDecStep);
   if (want > most) want = most;
   if (want > kDecMaxSplits) want = kDecMaxSplits;
   if (want < 1) want = 1;
