@@ -112,3 +112,17 @@ def test_other_calls_stay_with_sdpa(hip_lib):
     seen = []
     torch.func.vmap(lambda x: (seen.append(decode_attn(x, k, v, 0.1)), x)[1])(torch.stack([q, q]))
     assert seen == [None]
+
+
+@pytest.mark.parametrize("which", ["q", "k", "v"])
+def test_negated_views_are_read_as_their_values(hip_lib, which):
+    """A view whose negation is put off (the imaginary part of a conjugate is one) is SDPA's."""
+    ops = dict(zip("qkv", qkv(8, 1, 4, 2, 200, 128, torch.float16)))
+    want, _ = sa.block_sparse_attention(None, *ops.values(), None, 0.1)
+    ops[which] = torch._neg_view(-ops[which])
+    got, _ = sa.block_sparse_attention(None, *ops.values(), None, 0.1)
+    # SDPA's rounding against the kernel's: P and the output once each, as in bound()
+    ref, mass = exact(*(t.resolve_neg() for t in ops.values()), 0.1)
+    for out in (got, want):         # the same values
+        assert ((out.double() - ref).abs() <= 4 * bound(ref, mass, torch.float16)).all()
+    assert decode_attn(*ops.values(), 0.1) is None

@@ -108,8 +108,8 @@ def attn_prepared(q, k, kv_idx, scale, out, workspace):
 
 
 def _unwatched(q, k, v):
-    """Whether a launch on the tensors' data pointers is all there is to a call: dense tensors,
-    outside autograd, autocast, tracing, modes and functional transforms."""
+    """Whether a launch on the tensors' data pointers is all there is to a call: dense tensors
+    whose memory holds their values (no negation put off in a view's flag), outside autograd, autocast, tracing, modes and functional transforms."""
     wrapped = torch._C._functorch.is_functorch_wrapped_tensor
     return not ((torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad))
                 or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
@@ -117,6 +117,7 @@ def _unwatched(q, k, v):
                 or torch._C._get_tracing_state() is not None
                 or wrapped(q) or wrapped(k) or wrapped(v)
                 or q.is_nested or k.is_nested or v.is_nested
+                or q.is_neg() or k.is_neg() or v.is_neg()
                 or not (q.layout is k.layout is v.layout is torch.strided))
 
 
