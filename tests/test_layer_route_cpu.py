@@ -133,3 +133,17 @@ def test_row_lists_as_wide_as_the_mask_keep_the_wavefronts(rec, D, widest):
         listed = (nb + (nb + 31) // 32 + 1) // 2 * 2 * 4 + 8 * nb
         fits = waves * ((listed + (0 if D == 128 else 128 * D)) + 15 & ~15) <= 160 * 1024
         assert fits == (nb == widest) or D == 128         # (there 1024 is a cap on the copy to LDS)
+
+
+def test_refused_call_caches_no_block_means(rec):
+    """k_pool_at holds means that were computed, never the buffer of a call that failed."""
+    q, k, _ = qkv()
+    sa.SEL.mode = "topk"
+    rec.on["ugbsa_block_summary_means"] = lambda *a: -1
+    with pytest.raises(AssertionError):
+        sa.select_mask_v1(q, k, 0.125, layer_idx=3)
+    assert sa.SEL.k_pool_at == {}
+    del rec.on["ugbsa_block_summary_means"]
+    sa.select_mask_v1(q, k, 0.125, layer_idx=3)
+    means = sa.SEL.k_pool_at[3]
+    assert rec.calls[1][1][12] == means.data_ptr() and means.shape == (1, 4, 32, 64)

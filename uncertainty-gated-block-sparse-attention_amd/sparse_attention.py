@@ -383,8 +383,9 @@ def select_mask_v1(query, key_states, scaling, sel: Selector = None, want_scores
     if mode == _capi.MODE_MEAN and M > 1 and layer_idx is not None:
         # the mean K of each block, repeat_kv'd, cached for later planners (:230-232)
         means = torch.empty(B, H, nb, D, dtype=query.dtype, device=dev)
-        sel.k_pool_at[layer_idx] = means
     planes = block_summary(key_states, mode, means)
+    if means is not None:
+        sel.k_pool_at[layer_idx] = means
     k_bud = min(int(max(min(sel.k_max, sel.budget_blocks), sel.k_min)), nb)
     router = sel.mode == "router"
     k_eff = max(1, min(int(sel.budget_blocks), nb - 1)) if router else 0
