@@ -126,3 +126,14 @@ def test_negated_views_are_read_as_their_values(hip_lib, which):
     for out in (got, want):         # the same values
         assert ((out.double() - ref).abs() <= 4 * bound(ref, mass, torch.float16)).all()
     assert decode_attn(*ops.values(), 0.1) is None
+
+
+def test_many_short_sequences_stay_with_sdpa(hip_lib):
+    def taken(H, Hk, N, B, D=256):
+        return decode_attn(*qkv(9, B, H, Hk, N, D, torch.bfloat16), 0.1) is not None
+    assert not taken(8, 8, 32, 128) and not taken(8, 8, 1, 128)
+    assert taken(8, 8, 33, 128) and taken(8, 8, 32, 127) and taken(8, 4, 32, 128) and taken(8, 8, 32, 128, 128)
+    q, k, v = qkv(9, 128, 8, 8, 32, 256, torch.bfloat16)
+    out, _ = sa.block_sparse_attention(None, q, k, v, None, 0.1)
+    ref, mass = exact(q, k, v, 0.1)
+    assert ((out.double() - ref).abs() <= 4 * bound(ref, mass, q.dtype)).all()   # SDPA's rounding

@@ -142,6 +142,13 @@ def decode_attn(q, k, v, scale):
             and v.shape == k.shape and 0 < B <= 65535 and 0 < H <= 65535 and Hk > 0
             and H % Hk == 0 and 0 < N < 1 << 30):
         return None
+    # Head_dim 256 holds one workgroup a CU: with one query head per KV head, four or more
+    # rounds of them and one key step each, the library's smaller kernel is faster (us, this
+    # kernel's / its, 2048 pairs of batch and head: 16 keys 23.1 / 13.3, 32 keys 24.1 / 18.9, 40
+    # keys 28.3 / 58.6; 512 pairs end before the host's 10 us either way, 6.7 / 5.2, and so do
+    # 2048 at head_dim 128, 7.6 / 6.2).
+    if D == 256 and N <= 32 and H == Hk and B * H >= 1024:
+        return None
     sq, sk, sv = q.stride(), k.stride(), v.stride()
     pq, pk, pv = q.data_ptr(), k.data_ptr(), v.data_ptr()
     device, index = q.device, q.get_device()
