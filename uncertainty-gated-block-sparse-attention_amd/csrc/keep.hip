@@ -9,38 +9,43 @@
 // — the per-row keep test of the reference kernel (:87-103), read by the
 // attention kernels once per block instead of once per row.
 //
-// One workgroup per tile, its four wavefronts a quarter of the tile's rows
-// each: a lane owns WB consecutive blocks (one WB-byte word per row, a quarter
-// tile's words requested together) and leaves its rows' bits of each block in
-// LDS, a fourth of the block's mask.  Then the workgroup compacts the section
-// 256 blocks at a time.  Latency-bound at the per-row lengths seen (64 to 512
-// blocks): a wavefront per tile, 8 rows at a time, took 23 us for 28 x 64 tiles
-// of 64 blocks, where 56 of its 64 lanes had no word, and 39 us for 8 x 157
-// tiles of 157 blocks a byte at a time; now 14 and 22 us.
+// One workgroup per tile, a wavefront per 8 of its rows (eight or four): a lane
+// owns WB consecutive blocks (one WB-byte word per row, the eight words requested
+// together) and leaves its rows' bits of each block in LDS, a byte of the block's
+// mask.  Then the workgroup compacts the section 64 blocks a wavefront at a time.
+// Latency-bound at the per-row lengths seen (64 to 512 blocks).  GPU us, 64-row
+// tiles, by a wavefront a tile (8 rows at a time, its 8-byte words leaving 56
+// lanes idle at 64 blocks) / four wavefronts of 16 rows / eight of 8: 28 heads x
+// 4K rows x 64 blocks 22.0 / 9.2 / 8.6; 8 x 10007 x 157 27.2 / 16.3 / 11.1; 40 x
+// 20000 x 313 325 / 364 / 225; 64 x 16384 x 256 96.7 / 102 / 92.5 (the 16 words
+// of 16 rows cost registers, three wavefronts a SIMD).  32-row tiles, with
+// four of 16 rows (two without rows) / four of 8: 40 x 6000 x 94 36.0 / 52.8 /
+// 22.5; 2 x 8 x 20000 x 313 111 / 190 / 69.
 #include "common.h"
 #include "launch.h"
 
 namespace ugbsa {
 
-constexpr int kKeepWaves = 4;
 constexpr int kKeepSection = 1024;    // blocks whose masks LDS holds at once
 
 // WB bytes (blocks) per lane and row: 8 or 4 where rows and the mask are
 // multiples of it and the row is long enough to give most lanes a word, else 1.
-template <int WB>
-__global__ __launch_bounds__(64 * kKeepWaves) void keep_kv_idx_kernel(
-    const uint8_t* __restrict__ keep, int M, int NB, int block_m, int Qt,
+// BM: rows per tile, 64 or 32.
+template <int WB, int BM>
+__global__ __launch_bounds__(8 * BM) void keep_kv_idx_kernel(
+    const uint8_t* __restrict__ keep, int M, int NB, int Qt,
     int32_t* __restrict__ kv_idx, uint64_t* __restrict__ rowmask, int32_t* __restrict__ counts) {
-  constexpr int RW = 64 / kKeepWaves;    // mask bits per wavefront
-  __shared__ __align__(8) uint16_t s_mask[kKeepSection][kKeepWaves];   // one uint64 per block
-  __shared__ int s_cnt[kKeepWaves];
+  constexpr int RW = 8, NW = BM / RW;    // rows per wavefront, wavefronts
+  using Mask = std::conditional_t<BM == 64, uint64_t, uint32_t>;
+  __shared__ __align__(8) uint8_t s_mask[kKeepSection][NW];   // one Mask per block
+  __shared__ int s_cnt[NW];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t unit = blockIdx.x;
   const int64_t bh = unit / Qt;
   const int t = static_cast<int>(unit % Qt);
-  const int rows = min(block_m, M - t * block_m);
-  const int r0 = wave * RW;              // wavefronts past block_m have no rows
-  const uint8_t* kb = keep + (bh * M + static_cast<int64_t>(t) * block_m + r0) * NB;
+  const int rows = min(BM, M - t * BM);
+  const int r0 = wave * RW;
+  const uint8_t* kb = keep + (bh * M + static_cast<int64_t>(t) * BM + r0) * NB;
   int32_t* out = kv_idx + unit * NB;
   uint64_t* rm = rowmask != nullptr ? rowmask + unit * NB : nullptr;
   const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -69,19 +74,19 @@ __global__ __launch_bounds__(64 * kKeepWaves) void keep_kv_idx_kernel(
         for (int i = 0; i < WB; ++i)
           mk[i] |= static_cast<uint32_t>(((w[r] >> (8 * i)) & 0xFFull) != 0) << r;
 #pragma unroll
-      for (int i = 0; i < WB; ++i) s_mask[c + i][wave] = static_cast<uint16_t>(mk[i]);
+      for (int i = 0; i < WB; ++i) s_mask[c + i][wave] = static_cast<uint8_t>(mk[i]);
     }
     __syncthreads();
-    for (int c = 0; c < n; c += 64 * kKeepWaves) {
+    for (int c = 0; c < n; c += 64 * NW) {
       const int i = c + threadIdx.x;
-      const uint64_t mask = i < n ? *reinterpret_cast<const uint64_t*>(s_mask[i]) : 0ull;
+      const uint64_t mask = i < n ? *reinterpret_cast<const Mask*>(s_mask[i]) : 0u;
       const uint64_t bal = __ballot(mask != 0ull);
       if (c > 0) __syncthreads();        // the counts of the step before are read
       if (lane == 0) s_cnt[wave] = __popcll(bal);
       __syncthreads();
       int pos = cnt + __popcll(bal & lt_mask);
 #pragma unroll
-      for (int v = 0; v < kKeepWaves; ++v) {
+      for (int v = 0; v < NW; ++v) {
         pos += v < wave ? s_cnt[v] : 0;
         cnt += s_cnt[v];
       }
@@ -91,25 +96,33 @@ __global__ __launch_bounds__(64 * kKeepWaves) void keep_kv_idx_kernel(
       }
     }
   }
-  for (int s = cnt + threadIdx.x; s < NB; s += 64 * kKeepWaves) {
+  for (int s = cnt + threadIdx.x; s < NB; s += 64 * NW) {
     out[s] = NB;
     if (rm != nullptr) rm[s] = 0ull;
   }
   if (threadIdx.x == 0) counts[unit] = cnt;
 }
 
-hipError_t launch_keep_kv_idx(const uint8_t* keep, int B, int H, int M, int NB, int block_m,
-                              int32_t* kv_idx, uint64_t* rowmask, int32_t* counts,
-                              hipStream_t stream) {
-  const int Qt = (M + block_m - 1) / block_m;
+template <int BM>
+static void launch_keep_t(const uint8_t* keep, int B, int H, int M, int NB, int32_t* kv_idx,
+                          uint64_t* rowmask, int32_t* counts, hipStream_t stream) {
+  const int Qt = (M + BM - 1) / BM;
   const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(B) * H * Qt));
   const uintptr_t at = reinterpret_cast<uintptr_t>(keep);
   if (NB % 8 == 0 && at % 8 == 0 && NB >= 256)
-    keep_kv_idx_kernel<8><<<grid, 64 * kKeepWaves, 0, stream>>>(keep, M, NB, block_m, Qt, kv_idx, rowmask, counts);
+    keep_kv_idx_kernel<8, BM><<<grid, 8 * BM, 0, stream>>>(keep, M, NB, Qt, kv_idx, rowmask, counts);
   else if (NB % 4 == 0 && at % 4 == 0 && NB >= 128)
-    keep_kv_idx_kernel<4><<<grid, 64 * kKeepWaves, 0, stream>>>(keep, M, NB, block_m, Qt, kv_idx, rowmask, counts);
+    keep_kv_idx_kernel<4, BM><<<grid, 8 * BM, 0, stream>>>(keep, M, NB, Qt, kv_idx, rowmask, counts);
   else
-    keep_kv_idx_kernel<1><<<grid, 64 * kKeepWaves, 0, stream>>>(keep, M, NB, block_m, Qt, kv_idx, rowmask, counts);
+    keep_kv_idx_kernel<1, BM><<<grid, 8 * BM, 0, stream>>>(keep, M, NB, Qt, kv_idx, rowmask, counts);
+}
+
+hipError_t launch_keep_kv_idx(const uint8_t* keep, int B, int H, int M, int NB, int block_m,
+                              int32_t* kv_idx, uint64_t* rowmask, int32_t* counts,
+                              hipStream_t stream) {
+  if (block_m == 64) launch_keep_t<64>(keep, B, H, M, NB, kv_idx, rowmask, counts, stream);
+  else if (block_m == 32) launch_keep_t<32>(keep, B, H, M, NB, kv_idx, rowmask, counts, stream);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
