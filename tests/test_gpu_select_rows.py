@@ -105,6 +105,17 @@ def test_keep_lists(hip_lib, nb, block_m):
             assert np.array_equal(masks[:, :, t], np.take_along_axis(pad, got[:, :, t], -1))
 
 
+def test_keep_lists_of_many_tiles(hip_lib):
+    """More tiles than one launch dimension holds at a workgroup each."""
+    B, H = 8700, 2000                                   # 17.4 million one-row tiles of two blocks
+    keep = torch.zeros(B, H, 1, 2, dtype=torch.bool, device=DEV)
+    keep[..., 1] = torch.arange(B * H, device=DEV).view(B, H, 1) % 3 == 0
+    kv, _, most = keep_kv_idx(keep, 64, want_rowmask=False)
+    on = keep[..., 1]
+    assert most == 1
+    assert torch.equal(kv[..., 0], torch.where(on, 1, 2).to(torch.int32)) and (kv[..., 1] == 2).all()
+
+
 @pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16), (256, torch.bfloat16)])
 def test_cached_block_means(hip_lib, D, dtype):
     """k_pool_at holds the means of the summary planes in the model's dtype, once per query head."""

@@ -33,14 +33,15 @@ constexpr int kKeepSection = 1024;    // blocks whose masks LDS holds at once
 // BM: rows per tile, 64 or 32.
 template <int WB, int BM>
 __global__ __launch_bounds__(8 * BM) void keep_kv_idx_kernel(
-    const uint8_t* __restrict__ keep, int M, int NB, int Qt,
+    const uint8_t* __restrict__ keep, int64_t tiles, int M, int NB, int Qt,
     int32_t* __restrict__ kv_idx, uint64_t* __restrict__ rowmask, int32_t* __restrict__ counts) {
   constexpr int RW = 8, NW = BM / RW;    // rows per wavefront, wavefronts
   using Mask = std::conditional_t<BM == 64, uint64_t, uint32_t>;
   __shared__ __align__(8) uint8_t s_mask[kKeepSection][NW];   // one Mask per block
   __shared__ int s_cnt[NW];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t unit = blockIdx.x;
+  const int64_t unit = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+  if (unit >= tiles) return;
   const int64_t bh = unit / Qt;
   const int t = static_cast<int>(unit % Qt);
   const int rows = min(BM, M - t * BM);
@@ -107,14 +108,17 @@ template <int BM>
 static void launch_keep_t(const uint8_t* keep, int B, int H, int M, int NB, int32_t* kv_idx,
                           uint64_t* rowmask, int32_t* counts, hipStream_t stream) {
   const int Qt = (M + BM - 1) / BM;
-  const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(B) * H * Qt));
+  const int64_t tiles = static_cast<int64_t>(B) * H * Qt;
+  // rows of 2^20 workgroups: a launch dimension holds less than 2^32 threads
+  const int64_t per_row = tiles < (1 << 20) ? tiles : 1 << 20;
+  const dim3 grid(static_cast<unsigned>(per_row), static_cast<unsigned>((tiles + per_row - 1) / per_row));
   const uintptr_t at = reinterpret_cast<uintptr_t>(keep);
   if (NB % 8 == 0 && at % 8 == 0 && NB >= 256)
-    keep_kv_idx_kernel<8, BM><<<grid, 8 * BM, 0, stream>>>(keep, M, NB, Qt, kv_idx, rowmask, counts);
+    keep_kv_idx_kernel<8, BM><<<grid, 8 * BM, 0, stream>>>(keep, tiles, M, NB, Qt, kv_idx, rowmask, counts);
   else if (NB % 4 == 0 && at % 4 == 0 && NB >= 128)
-    keep_kv_idx_kernel<4, BM><<<grid, 8 * BM, 0, stream>>>(keep, M, NB, Qt, kv_idx, rowmask, counts);
+    keep_kv_idx_kernel<4, BM><<<grid, 8 * BM, 0, stream>>>(keep, tiles, M, NB, Qt, kv_idx, rowmask, counts);
   else
-    keep_kv_idx_kernel<1, BM><<<grid, 8 * BM, 0, stream>>>(keep, M, NB, Qt, kv_idx, rowmask, counts);
+    keep_kv_idx_kernel<1, BM><<<grid, 8 * BM, 0, stream>>>(keep, tiles, M, NB, Qt, kv_idx, rowmask, counts);
 }
 
 hipError_t launch_keep_kv_idx(const uint8_t* keep, int B, int H, int M, int NB, int block_m,
