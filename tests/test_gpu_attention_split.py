@@ -81,3 +81,26 @@ def test_offsets_far_apart(hip_lib, D):
         kv[0, :, t, :t + 1] = torch.arange(t + 1, dtype=torch.int32)
     out = block_sparse_attn_v2(q.to(DEV), k.to(DEV), v.to(DEV), kv.to(DEV), D ** -0.5)
     check(out, OA.gathered_attention(f32np(q), f32np(k), f32np(v), kv.numpy(), D ** -0.5))
+
+
+# past 512 blocks, where only head_dim 64 splits: lists of none to 40 blocks, a ragged last tile
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H", [1, 2])
+def test_long_context_of_few_tiles(hip_lib, D, H):
+    print(f"[case] split lists past 512 blocks D={D} H={H}", flush=True)
+    M = 64 * 530 - 9
+    q, k, v = qkv(M + D + H, 1, H, 1, M, D, torch.bfloat16)
+    nb = qt = 530
+    g = torch.Generator().manual_seed(H)
+    kv = torch.full((1, H, qt, 40), nb, dtype=torch.int32)
+    for h in range(H):
+        for t in range(qt):
+            n = min((h + t) % 41, t + 1)
+            kv[0, h, t, torch.randperm(40, generator=g)[:n]] = torch.randperm(t + 1, generator=g)[:n].to(torch.int32)
+    ref = OA.gathered_attention(f32np(q), f32np(k), f32np(v), kv.numpy(), D ** -0.5)
+    qd, kd, vd = q.to(DEV), k.to(DEV), v.to(DEV)
+    check(block_sparse_attn_v2(qd, kd, vd, kv.to(DEV), D ** -0.5), ref)
+    # the same lists as row masks that every row of a tile shares
+    keep = torch.zeros(1, H, qt, nb + 1, dtype=torch.bool).scatter_(3, kv.long(), True)[..., :nb]
+    keep = keep.repeat_interleave(64, dim=2)[:, :, :M].contiguous()
+    check(block_sparse_attn(qd, kd, vd, keep.to(DEV), D ** -0.5), ref)

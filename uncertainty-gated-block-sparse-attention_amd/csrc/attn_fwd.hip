@@ -244,17 +244,27 @@ static int pipe_slots(int D) { return D == 64 ? 2048 : 1024; }
 // 272, 240), 64 of 10K 144 (1; 155, 170); head_dim 64, 8 heads, 157 of 10K 147
 // (4; 249, 173), 16 heads, 32 of 8K 89 (1; 103, 103).
 static int attn_split(int64_t tiles, int Qt, int k_slots, int NB, int D, bool rowmask) {
-  if (NB > kGenBlocks || (D > 128 && rowmask)) return 1;   // (attn_pipe.h: no such instance)
+  // Past kGenBlocks only at head_dim 64: its two wavefronts per SIMD leave half of
+  // them idle, or two long lists on one, in calls of fewer tiles than they are
+  // (1 / 2 / 4 wavefronts, lists of up to 256: 1 head, 516 blocks 358 / 211 / 128
+  // us, 2048 blocks 629 / 528 / 522; 2 heads, 750 blocks 491 / 311 / 273; one
+  // wavefront per SIMD took 331, 559 and 338).
+  if (NB > kGenBlocks && D > 64) return 1;
+  if (D > 128 && rowmask) return 1;                        // (attn_pipe.h: no such instance)
   const int64_t most = k_slots < Qt ? k_slots : Qt;             // longest list
   const double mean = most - 0.5 * most * (most - 1) / Qt;      // sum of min(t + 1, most) / Qt
   const double gain = D > 128 ? 0.75 : 0.93;
   int best = 1;
   double best_t = 0.0;
   for (int s = 1; s <= 4; s *= 2) {
-    if (s * pipe_wave_lds(D, 4, D != 128, k_slots, NB, rowmask) > 160 * 1024) break;
+    // wavefronts the chip holds: long lists leave a CU's LDS room for fewer
+    const int wave_lds = pipe_wave_lds(D, 4, D != 128, k_slots, NB, rowmask);
+    const int fit = 256 * (160 * 1024 / (s * wave_lds)) * s;
+    if (fit == 0) break;
+    const int slots = fit < pipe_slots(D) ? fit : pipe_slots(D);
     const double fixed = s == 1 ? 6.0 : 8.0;
     const double longest = fixed + static_cast<double>(most) / s;
-    const double all = tiles * (fixed * s + mean) / pipe_slots(D);
+    const double all = tiles * (fixed * s + mean) / slots;
     const double t = (longest > all ? longest : all) + 0.25 * longest;
     if (s == 1 || t < gain * best_t) { best = s; best_t = t; }
   }
@@ -550,8 +560,12 @@ static hipError_t launch_attn_fwd_e(const uint16_t* q, int64_t sq_b, int64_t sq_
     const int32_t* tile_order = nullptr;
     // Not ranked: calls whose wavefronts all start at once, and row-masked calls
     // in one launch, whose lists are unions over 64 rows and so grow with t (the
-    // two ranking launches are 10 us of a 241 us layer of 28 heads x 4K).
-    if (order_ws != nullptr && tiles * split > pipe_slots(D) &&
+    // two ranking launches are 10 us of a 241 us layer of 28 heads x 4K).  Ranked
+    // all the same: long contexts at head_dim 64 whose wavefronts all start at once
+    // but share SIMDs, unless every list is short (2 heads x 1024 blocks, lists of
+    // up to 64 / 32: 154 / 94 us unranked, 130 / 102 ranked).
+    const bool shared = D == 64 && NBk > kGenBlocks && k_slots > 32 && tiles * split > 1024;
+    if (order_ws != nullptr && (tiles * split > pipe_slots(D) || shared) &&
         (rowmask == nullptr || NBk > kGenBlocks)) {
       hipError_t e = launch_attn_tile_order(kv_idx, si_b, si_h, si_t, B, H, Qt, k_slots, NBk,
                                             order_ws, stream);
