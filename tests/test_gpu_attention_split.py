@@ -104,3 +104,33 @@ def test_long_context_of_few_tiles(hip_lib, D, H):
     keep = torch.zeros(1, H, qt, nb + 1, dtype=torch.bool).scatter_(3, kv.long(), True)[..., :nb]
     keep = keep.repeat_interleave(64, dim=2)[:, :, :M].contiguous()
     check(block_sparse_attn(qd, kd, vd, keep.to(DEV), D ** -0.5), ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kept", [1500, 1600])
+def test_long_row_lists(hip_lib, dtype, kept):
+    """Head_dim 64, row-masked lists on either side of the length (1575 slots) where another form
+    of the kernel takes over; the tiles that hold them and some others against fp32."""
+    print(f"[case] long row lists {dtype} kept={kept}", flush=True)
+    nb, D = 1610, 64
+    M = 64 * nb - 30
+    q, k, v = (t.to(DEV) for t in qkv(kept, 1, 2, 1, M, D, dtype))
+    g = torch.Generator(device=DEV).manual_seed(kept)
+    tile = torch.arange(M, device=DEV) // 64
+    keep = torch.rand(1, 2, M, nb, device=DEV, generator=g) < 0.004
+    keep[0, :, torch.arange(M, device=DEV), tile] = True
+    full = (1605, nb - 1)                                   # whole and ragged tiles with long lists
+    for t in full:
+        rows = slice(64 * t, min(M, 64 * t + 64))
+        keep[0, :, rows, :kept - 1] |= torch.rand(M, device=DEV, generator=g)[rows, None] < 0.7
+        keep[0, :, rows, kept - 1:t] = False
+    keep = keep & (torch.arange(nb, device=DEV) <= tile[:, None])
+    out = block_sparse_attn(q, k, v, keep, D ** -0.5).float()
+    for h in range(2):
+        for t in (0, 1, 700, 1604) + full:
+            rows = slice(64 * t, min(M, 64 * t + 64))
+            s = (q[0, h, rows].float() @ k[0, 0].float().t().contiguous()) * D ** -0.5
+            on = keep[0, h, rows].repeat_interleave(64, dim=1)[:, :M]
+            on = on & (torch.arange(M, device=DEV) <= torch.arange(M, device=DEV)[rows, None])
+            want = torch.softmax(s.masked_fill(~on, float("-inf")), -1) @ v[0, 0].float()
+            check(out[0, h, rows], f32np(want))

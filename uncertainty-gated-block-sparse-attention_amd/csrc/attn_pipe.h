@@ -76,7 +76,7 @@ constexpr int cfg_nt(int cfg) { return cfg % 16; }
 constexpr int cfg_split(int cfg) { return cfg / 16 % 16 + 1; }
 
 template <typename E, int D, int CFG, bool QLDS, bool SB, bool OA>
-__global__ __launch_bounds__(64 * (4 / cfg_nt(CFG)) * cfg_split(CFG), D == 64 ? 2 : 1) void attn_fwd_pipe_kernel(
+__global__ __launch_bounds__(64 * (4 / cfg_nt(CFG)) * cfg_split(CFG), D == 64 && QLDS ? 2 : 1) void attn_fwd_pipe_kernel(
     const uint16_t* __restrict__ q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
     const uint16_t* __restrict__ k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
     const uint16_t* __restrict__ vt, const int32_t* __restrict__ kv_idx,
