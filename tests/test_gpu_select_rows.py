@@ -54,6 +54,16 @@ def test_belief_mass_never_reached(hip_lib, nb, k_max, top_p):
     assert res.keep[0, 0, 0].sum() == k_max        # one visible block, the rest lowest first
 
 
+# the sort sizes (64, 128, 256, 512 keys) on either side of each, rows of fewer blocks among them
+@pytest.mark.parametrize("k_max", [64, 65, 128, 129, 256, 257, 400])
+def test_belief_sort_sizes(hip_lib, k_max):
+    print(f"[case] belief sort k_max={k_max}", flush=True)
+    g = torch.Generator().manual_seed(k_max)
+    q = torch.randn(1, 1, 64 * 300, 64, generator=g).to(torch.bfloat16)
+    k = (0.2 * torch.randn(1, 1, 64 * 300, 64, generator=g)).to(torch.bfloat16)
+    check("belief", dict(top_p=0.8, k_min=1, k_max=k_max), q, k)
+
+
 @pytest.mark.parametrize("nb", [40, 100, 300])
 @pytest.mark.parametrize("mode,kw", [("topk", dict(budget_blocks=16)),
                                      ("router", dict(budget_blocks=24))])

@@ -23,7 +23,7 @@
 //
 // 28 heads x 4096 rows x 64 blocks: 35 us (a radix select through LDS
 // histograms, a 64-bit sort and LDS flags took 119); 8 x 10007 x 157, belief:
-// 90 us (117).
+// 87 us (117).
 #include "common.h"
 #include "launch.h"
 
@@ -56,12 +56,12 @@ __device__ __forceinline__ KeyCut key_cut(const uint32_t (&key)[RK], int K) {
   return r;
 }
 
-// Descending bitonic sort of KP keys, element e = lane + 64 r.
-template <int KP>
-__device__ __forceinline__ void sort_keys(uint32_t (&v)[KP / 64], int lane) {
+// Descending bitonic sort of the first KP keys of v, element e = lane + 64 r.
+template <int KP, int RT>
+__device__ __forceinline__ void bitonic_keys(uint32_t (&v)[RT], int lane) {
   constexpr int R = KP / 64;
-  constexpr int LOG_KP = KP == 64 ? 6 : KP == 128 ? 7 : 9;
-  static_assert((1 << LOG_KP) == KP, "KP is a power of two");
+  constexpr int LOG_KP = KP == 64 ? 6 : KP == 128 ? 7 : KP == 256 ? 8 : 9;
+  static_assert((1 << LOG_KP) == KP && R <= RT, "KP is a power of two within v");
   static_for<LOG_KP>([&](auto lk) {
     constexpr int kk = 2 << decltype(lk)::value;
     static_for<decltype(lk)::value + 1>([&](auto lj) {
@@ -80,6 +80,19 @@ __device__ __forceinline__ void sort_keys(uint32_t (&v)[KP / 64], int lane) {
       for (int r = 0; r < R; ++r) v[r] = nv[r];
     });
   });
+}
+
+// Sorts the n keys of v (the rest are 0), as few of its registers as hold them
+// (rows of up to 64 blocks have a body of their own).
+template <int KP>
+__device__ __forceinline__ void sort_keys(uint32_t (&v)[KP / 64], int n, int lane) {
+  if constexpr (KP > 128) {
+    if (n <= 128) return bitonic_keys<128>(v, lane);
+  }
+  if constexpr (KP > 256) {
+    if (n <= 256) return bitonic_keys<256>(v, lane);
+  }
+  bitonic_keys<KP>(v, lane);
 }
 
 // Key of rank e (0 = best) of a sorted v.
@@ -118,7 +131,7 @@ __device__ __forceinline__ int belief_count(const RowsArgs& a, const float (&x)[
 #pragma unroll
   for (int r = 0; r < R; ++r) v[r] = lane + 64 * r < n_sel ? cand[lane + 64 * r] : 0u;
   wave_lds_sync();
-  sort_keys<KP>(v, lane);
+  sort_keys<KP>(v, n_sel, lane);
 
   // softmax over the visible blocks (max-subtracted, fp32), then the
   // cumulative mass of the sorted probabilities
@@ -319,8 +332,16 @@ __device__ __forceinline__ void rows_body(const RowsArgs& a, int64_t bh, int row
   }
 }
 
+// Wavefronts per SIMD: the belief body's keys and scores of long rows would leave
+// one or two. Held to two at 64 keys a lane it spills 28-68 bytes and is the
+// faster all the same (1 head x 200K tokens 5.29 -> 3.84 ms; three at 32, 2 heads x
+// 131K 2.19 -> 1.77).
+constexpr int rows_eu_waves(int rkmax, bool belief) {
+  return !belief ? 1 : rkmax == 64 ? 2 : rkmax == 32 ? 3 : 1;
+}
+
 template <int RKMAX, bool BELIEF, int KP>
-__global__ __launch_bounds__(64 * kRowsWaves) void select_rows_kernel(const RowsArgs a) {
+__global__ __launch_bounds__(64 * kRowsWaves, rows_eu_waves(RKMAX, BELIEF)) void select_rows_kernel(const RowsArgs a) {
   __shared__ uint32_t s_cand[BELIEF ? kRowsWaves * KP : 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // one wave-uniform group of rows: row indices and branches stay scalar
@@ -377,8 +398,12 @@ static hipError_t launch_rows_k(const RowsArgs& a, hipStream_t stream) {
 hipError_t launch_select_rows(const RowsArgs& a, hipStream_t stream) {
   if (a.K > 512 || a.nrows % kBlock != 0) return hipErrorInvalidValue;
   if (!a.belief) return launch_rows_k<false, 64>(a, stream);
-  // (the default k_max, 112, sorts 128 keys)
+  // as many sorted keys as ranks are asked for (the default k_max, 112: 128): 8
+  // heads x 10007 rows, k_max 200: 223 us with 512, 131 with 256; k_max 40: 111
+  // with 128, 98 with 64
+  if (a.K <= 64) return launch_rows_k<true, 64>(a, stream);
   if (a.K <= 128) return launch_rows_k<true, 128>(a, stream);
+  if (a.K <= 256) return launch_rows_k<true, 256>(a, stream);
   return launch_rows_k<true, 512>(a, stream);
 }
 
