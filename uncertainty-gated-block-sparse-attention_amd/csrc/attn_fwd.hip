@@ -255,16 +255,17 @@ static bool long_row_lists(int D, int k_slots, int NB, bool rowmask) {
 // (4; 249, 173), 16 heads, 32 of 8K 89 (1; 103, 103).
 static int attn_split(int64_t tiles, int Qt, int k_slots, int NB, int D, bool rowmask) {
   // Past kGenBlocks only at head_dim 64: its two wavefronts per SIMD leave half of
-  // them idle, or two long lists on one, in calls of fewer tiles than they are
-  // (1 / 2 / 4 wavefronts, lists of up to 256: 1 head, 516 blocks 358 / 211 / 128
-  // us, 2048 blocks 629 / 528 / 522; 2 heads, 750 blocks 491 / 311 / 273; one
-  // wavefront per SIMD took 331, 559 and 338).
+  // them idle, or two long lists on one, in calls of few tiles (1 / 2 / 4
+  // wavefronts, lists of up to 256: 1 head, 516 blocks 358 / 211 / 128 us, 1536
+  // blocks 538 / 352 / 356; 2 heads, 750 blocks 491 / 311 / 273; one wavefront per
+  // SIMD took 331, 357 and 338).  There for at least 15 %: 1 head on the full list
+  // of 3125 blocks, which the rule puts 8 % ahead with two, 6.3 ms, with two 7.5.
   if (NB > kGenBlocks && D > 64) return 1;
   // (attn_pipe.h: no such instances)
   if ((D > 128 && rowmask) || long_row_lists(D, k_slots, NB, rowmask)) return 1;
   const int64_t most = k_slots < Qt ? k_slots : Qt;             // longest list
   const double mean = most - 0.5 * most * (most - 1) / Qt;      // sum of min(t + 1, most) / Qt
-  const double gain = D > 128 ? 0.75 : 0.93;
+  const double gain = D > 128 ? 0.75 : NB > kGenBlocks ? 0.85 : 0.93;
   int best = 1;
   double best_t = 0.0;
   for (int s = 1; s <= 4; s *= 2) {
