@@ -134,3 +134,22 @@ def test_long_row_lists(hip_lib, dtype, kept):
             on = on & (torch.arange(M, device=DEV) <= torch.arange(M, device=DEV)[rows, None])
             want = torch.softmax(s.masked_fill(~on, float("-inf")), -1) @ v[0, 0].float()
             check(out[0, h, rows], f32np(want))
+
+
+@pytest.mark.parametrize("slots", [4600, 4800])
+def test_long_plain_lists(hip_lib, slots):
+    """Head_dim 64, lists on either side of the length (4700 slots) where that form takes over, their
+    blocks anywhere among the sentinels."""
+    print(f"[case] long plain lists slots={slots}", flush=True)
+    M, D = 64 * 40 - 7, 64
+    q, k, v = qkv(slots, 1, 2, 1, M, D, torch.bfloat16)
+    g = torch.Generator().manual_seed(slots)
+    short = torch.full((1, 2, 40, 40), 40, dtype=torch.int32)
+    kv = torch.full((1, 2, 40, slots), 40, dtype=torch.int32)
+    for h in range(2):
+        for t in range(40):
+            pick = torch.randperm(t + 1, generator=g)[:(7 * t + h) % (t + 2)].to(torch.int32)
+            short[0, h, t, :len(pick)] = pick
+            kv[0, h, t, torch.randperm(slots, generator=g)[:len(pick)]] = pick
+    out = block_sparse_attn_v2(q.to(DEV), k.to(DEV), v.to(DEV), kv.to(DEV), D ** -0.5)
+    check(out, OA.gathered_attention(f32np(q), f32np(k), f32np(v), short.numpy(), D ** -0.5))

@@ -228,14 +228,15 @@ int attn_wave_lds(int N, int D, int k_slots, bool row_masks) {
 // 256 CUs, two at head_dim 64.
 static int pipe_slots(int D) { return D == 64 ? 2048 : 1024; }
 
-// Head_dim 64 keeps Q in LDS so that two wavefronts share a SIMD; row-masked lists
-// of more than 1575 slots (12 bytes each) leave a CU room for fewer than six such
-// wavefronts, and then the form of one wavefront per SIMD, with Q in registers and
-// two K / V^T sets, is the faster one: 8 heads x 131K tokens, a quarter of the
-// cells triggered 35.7 / 25.4 ms, budget 64 27.0 / 23.4; at 98K tokens, where six
-// fit, 14.0 / 14.3 and 13.7 / 13.7.
-static bool long_row_lists(int D, int k_slots, int NB, bool rowmask) {
-  return D == 64 && rowmask && 6 * pipe_wave_lds(64, 4, true, k_slots, NB, true) > 160 * 1024;
+// Head_dim 64 keeps Q in LDS so that two wavefronts share a SIMD; beside lists of
+// more than 1575 slots with masks (12 bytes a slot), or 4700 without, fewer than
+// six such wavefronts fit a CU, and then the form of one wavefront per SIMD, with Q
+// in registers and two K / V^T sets, is the faster one: row masks, 8 heads x 131K
+// tokens, a quarter of the cells triggered 35.7 / 25.4 ms, budget 64 27.0 / 23.4
+// (98K tokens, where six fit, 14.0 / 14.3 and 13.7 / 13.7); one head on the full
+// causal list, 524K tokens 71.7 / 43.1, 300K 16.4 / 14.6.
+static bool long_lists(int D, int k_slots, int NB, bool rowmask) {
+  return D == 64 && 6 * pipe_wave_lds(64, 4, true, k_slots, NB, rowmask) > 160 * 1024;
 }
 
 // Wavefronts per 64-row tile.  A tile is a chain of its listed blocks, so a
@@ -262,7 +263,7 @@ static int attn_split(int64_t tiles, int Qt, int k_slots, int NB, int D, bool ro
   // of 3125 blocks, which the rule puts 8 % ahead with two, 6.3 ms, with two 7.5.
   if (NB > kGenBlocks && D > 64) return 1;
   // (attn_pipe.h: no such instances)
-  if ((D > 128 && rowmask) || long_row_lists(D, k_slots, NB, rowmask)) return 1;
+  if ((D > 128 && rowmask) || long_lists(D, k_slots, NB, rowmask)) return 1;
   const int64_t most = k_slots < Qt ? k_slots : Qt;             // longest list
   const double mean = most - 0.5 * most * (most - 1) / Qt;      // sum of min(t + 1, most) / Qt
   const double gain = D > 128 ? 0.75 : NB > kGenBlocks ? 0.85 : 0.93;
@@ -592,10 +593,12 @@ static hipError_t launch_attn_fwd_e(const uint16_t* q, int64_t sq_b, int64_t sq_
       return launch_attn_pipe<E, 128, 4, false, false>(q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx,
                                           rowmask, si_b, si_h, si_t, B, H, Hk, M, N, Qt, k_slots,
                                           scale, out, so_b, so_h, so_m, stream, tile_order, split);
-    if (long_row_lists(D, k_slots, NBk, rowmask != nullptr))
-      return launch_attn_pipe_t<E, 64, 4, false, false, false, 1, true>(
-          q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx, rowmask, si_b, si_h, si_t, B, H, Hk,
-          M, N, Qt, k_slots, scale, out, so_b, so_h, so_m, stream, tile_order);
+    if (long_lists(D, k_slots, NBk, rowmask != nullptr)) {
+      auto* launch = rowmask != nullptr ? launch_attn_pipe_t<E, 64, 4, false, false, false, 1, true>
+                                        : launch_attn_pipe_t<E, 64, 4, false, false, false, 1, false>;
+      return launch(q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx, rowmask, si_b, si_h, si_t,
+                    B, H, Hk, M, N, Qt, k_slots, scale, out, so_b, so_h, so_m, stream, tile_order);
+    }
     return launch_attn_pipe<E, 64, 4, true, true>(q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx,
                                        rowmask, si_b, si_h, si_t, B, H, Hk, M, N, Qt, k_slots,
                                        scale, out, so_b, so_h, so_m, stream, tile_order, split);
