@@ -210,6 +210,18 @@ int ugbsa_attn_fwd_rows(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
                         void* out, int64_t so_b, int64_t so_h, int64_t so_m, int64_t so_d,
                         void* workspace, int64_t workspace_elems, void* stream);
 
+/* ugbsa_attn_fwd_rows for lists that grow with the tile, as those of
+ * ugbsa_select_mask's rows do: tiles are taken by descending index where that
+ * saves ranking them by their work.  The result is the same for any lists. */
+int ugbsa_attn_fwd_rows_grow(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m, int64_t sq_d,
+                             const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n, int64_t sk_d,
+                             const void* v, int64_t sv_b, int64_t sv_h, int64_t sv_n, int64_t sv_d,
+                             const int32_t* kv_idx, const uint64_t* rowmask, int64_t si_b,
+                             int64_t si_h, int64_t si_t, int64_t si_s, int B, int H, int Hk, int M,
+                             int N, int D, int dtype, int Qt, int k_slots, int block_m, float scale,
+                             void* out, int64_t so_b, int64_t so_h, int64_t so_m, int64_t so_d,
+                             void* workspace, int64_t workspace_elems, void* stream);
+
 /* LDS bytes that one wavefront of the 64-row-tile attention takes for Q, the
  * list of a tile of k_slots slots and (row_masks != 0) its masks. */
 int64_t ugbsa_attn_wave_lds(int N, int D, int k_slots, int row_masks);

@@ -153,3 +153,17 @@ def test_long_plain_lists(hip_lib, slots):
             kv[0, h, t, torch.randperm(slots, generator=g)[:len(pick)]] = pick
     out = block_sparse_attn_v2(q.to(DEV), k.to(DEV), v.to(DEV), kv.to(DEV), D ** -0.5)
     check(out, OA.gathered_attention(f32np(q), f32np(k), f32np(v), short.numpy(), D ** -0.5))
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_tile_order_of_row_masks(hip_lib, D):
+    """Tiles ranked by their work or by descending index: the same bits, lists that do not grow."""
+    H, M = 40, 64 * 60 - 11                             # 2400 tiles, more than start at once
+    q, k, v = (t.to(DEV) for t in qkv(D, 1, H, 4, M, D, torch.bfloat16))
+    tile, nbs = torch.arange(M, device=DEV) // 64, torch.arange(60, device=DEV)
+    keep = (tile[:, None] == nbs) | ((tile % 8 == 1)[:, None] & (nbs <= tile[:, None]))
+    keep = keep.expand(1, H, M, 60).contiguous()
+    ranked = block_sparse_attn(q, k, v, keep, D ** -0.5)
+    assert torch.equal(ranked, block_sparse_attn(q, k, v, keep, D ** -0.5, lists_grow=True))
+    check(ranked[:, :1], OA.keep_attention(f32np(q[:, :1]), f32np(k[:, :1]), f32np(v[:, :1]),
+                                           keep[:, :1].cpu().numpy(), D ** -0.5))

@@ -147,3 +147,22 @@ def test_refused_call_caches_no_block_means(rec):
     sa.select_mask_v1(q, k, 0.125, layer_idx=3)
     means = sa.SEL.k_pool_at[3]
     assert rec.calls[1][1][12] == means.data_ptr() and means.shape == (1, 4, 32, 64)
+
+
+def test_row_masked_calls_say_whether_their_lists_grow(rec, monkeypatch):
+    """A per-row layer's lists do; a caller's own masks may be any, so its tiles are ranked."""
+    q, k, v = qkv()
+    sa.SEL.kernel_v2 = False
+    module = type("Layer", (), {"layer_idx": 0})
+    keep = torch.zeros(1, 4, 2048, 32, dtype=torch.bool).as_subclass(Dev)
+    monkeypatch.setattr(sa, "_block_select_mask", lambda *a: keep)
+    sa.block_sparse_attention(module, q, k, v, None, 0.125)
+    assert "ugbsa_attn_fwd_rows_grow" in rec.names() and "ugbsa_attn_fwd_rows" not in rec.names()
+    rec.calls.clear()
+    block_sparse_attn(q, k, v, keep, 0.125)
+    assert "ugbsa_attn_fwd_rows" in rec.names()
+    seen = []
+    monkeypatch.setattr(sa, "block_sparse_attn",
+                        lambda q, k, v, keep, scale, block_n, out, workspace: seen.append(1))
+    sa.block_sparse_attention(module, q, k, v, None, 0.125)
+    assert seen == [1]

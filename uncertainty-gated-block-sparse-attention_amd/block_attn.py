@@ -213,14 +213,16 @@ def _list_as_wide_as_mask(N, D, NB, block_m):
 
 
 def block_sparse_attn(q, k, v, keep, scale, block_n=64, block_m=64,
-                      num_warps=4, num_stages=1, out=None, workspace=None):
+                      num_warps=4, num_stages=1, out=None, workspace=None, lists_grow=False):
     """Per-row-selection block-sparse causal attention (HIP, bf16 / fp16 MFMA).
 
     q : [B, H, M, D] bf16 or fp16; k, v : [B, Hk, N, D] in q's dtype; keep : [B, H, M, NB]
     bool (True = the row attends to the block).  Same contract as
     src/triton_block_attn.py:149-182: per Q tile the union of its rows'
     blocks is visited in ascending order (``_compute_kv_idx``) and each row
-    only sees the keys of its own kept blocks, causally.
+    only sees the keys of its own kept blocks, causally.  ``lists_grow``: later
+    tiles keep about as many blocks as earlier ones or more, as the per-row
+    selector's do (a matter of speed alone).
     """
     assert q.dim() == 4 and k.shape == v.shape and q.shape[0] == k.shape[0] \
         and q.shape[-1] == k.shape[-1], "q [B,H,M,D], k = v [B,Hk,N,D] expected"
@@ -244,7 +246,8 @@ def block_sparse_attn(q, k, v, keep, scale, block_n=64, block_m=64,
     assert out.shape == q.shape and out.dtype == q.dtype and out.stride(-1) == 1
     if workspace is None:
         workspace = attn_workspace(B, Hk, N, D, q.device, q.dtype)
-    rc = _capi.lib().ugbsa_attn_fwd_rows(
+    lib = _capi.lib()
+    rc = (lib.ugbsa_attn_fwd_rows_grow if lists_grow else lib.ugbsa_attn_fwd_rows)(
         q.data_ptr(), *q.stride(),
         k.data_ptr(), *k.stride(),
         v.data_ptr(), *v.stride(),

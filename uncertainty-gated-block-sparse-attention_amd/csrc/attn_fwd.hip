@@ -564,22 +564,24 @@ static hipError_t launch_attn_fwd_e(const uint16_t* q, int64_t sq_b, int64_t sq_
                                     int N, int D, int Qt, int k_slots, int block_m, float scale,
                                     uint16_t* out, int64_t so_b, int64_t so_h, int64_t so_m,
                                     hipStream_t stream, const uint64_t* rowmask,
-                                    int32_t* order_ws) {
+                                    int32_t* order_ws, bool lists_grow) {
   if (uses_pipe(D, block_m)) {   // the pipelined kernel (its K/V operand layout is prepared)
     if (k_slots > kPipeMaxSlots) return hipErrorInvalidValue;
     const int NBk = (N + kBlock - 1) / kBlock;
     const int64_t tiles = static_cast<int64_t>(B) * H * Qt;
     const int split = attn_split(tiles, Qt, k_slots, NBk, D, rowmask != nullptr);
     const int32_t* tile_order = nullptr;
-    // Not ranked: calls whose wavefronts all start at once, and row-masked calls
-    // in one launch, whose lists are unions over 64 rows and so grow with t (the
-    // two ranking launches are 10 us of a 241 us layer of 28 heads x 4K).  Ranked
-    // all the same: long contexts at head_dim 64 whose wavefronts all start at once
-    // but share SIMDs, unless every list is short (2 heads x 1024 blocks, lists of
-    // up to 64 / 32: 154 / 94 us unranked, 130 / 102 ranked).
+    // Not ranked: calls whose wavefronts all start at once, and calls in one launch
+    // whose caller knows that the lists grow with t, as the per-row selector's unions
+    // over 64 rows do (the two ranking launches are 10 us of a 241 us layer of 28
+    // heads x 4K; of other row masks, every 8th tile dense, 28 heads x 16K take 576 us
+    // unranked, 485 ranked).  Ranked all the same: long contexts at head_dim 64 whose
+    // wavefronts all start at once but share SIMDs, unless every list is short (2
+    // heads x 1024 blocks, lists of up to 64 / 32: 154 / 94 us unranked, 130 / 102
+    // ranked).
     const bool shared = D == 64 && NBk > kGenBlocks && k_slots > 32 && tiles * split > 1024;
     if (order_ws != nullptr && (tiles * split > pipe_slots(D) || shared) &&
-        (rowmask == nullptr || NBk > kGenBlocks)) {
+        (!lists_grow || NBk > kGenBlocks)) {
       hipError_t e = launch_attn_tile_order(kv_idx, si_b, si_h, si_t, B, H, Qt, k_slots, NBk,
                                             order_ws, stream);
       if (e != hipSuccess) return e;
@@ -623,14 +625,17 @@ hipError_t launch_attn_fwd(const uint16_t* q, int64_t sq_b, int64_t sq_h, int64_
                            int64_t si_h, int64_t si_t, int B, int H, int Hk, int M, int N,
                            int D, int elem, int Qt, int k_slots, int block_m, float scale,
                            uint16_t* out, int64_t so_b, int64_t so_h, int64_t so_m,
-                           hipStream_t stream, const uint64_t* rowmask, int32_t* order_ws) {
+                           hipStream_t stream, const uint64_t* rowmask, int32_t* order_ws,
+                           bool lists_grow) {
   if (elem == ElemF16::code)
     return launch_attn_fwd_e<ElemF16>(q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx, si_b,
                                       si_h, si_t, B, H, Hk, M, N, D, Qt, k_slots, block_m, scale,
-                                      out, so_b, so_h, so_m, stream, rowmask, order_ws);
+                                      out, so_b, so_h, so_m, stream, rowmask, order_ws,
+                                      lists_grow);
   return launch_attn_fwd_e<ElemBf16>(q, sq_b, sq_h, sq_m, k, sk_b, sk_h, sk_n, vt, kv_idx, si_b,
                                      si_h, si_t, B, H, Hk, M, N, D, Qt, k_slots, block_m, scale,
-                                     out, so_b, so_h, so_m, stream, rowmask, order_ws);
+                                     out, so_b, so_h, so_m, stream, rowmask, order_ws,
+                                     lists_grow);
 }
 
 }  // namespace ugbsa

@@ -370,7 +370,7 @@ int attn_fwd_common(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m, int
                     int64_t si_t, int64_t si_s, int B, int H, int Hk, int M, int N, int D,
                     int dtype, int Qt, int k_slots, int block_m, float scale, void* out,
                     int64_t so_b, int64_t so_h, int64_t so_m, int64_t so_d, void* workspace,
-                    int64_t workspace_elems, void* stream) {
+                    int64_t workspace_elems, void* stream, bool lists_grow = false) {
   int rc = check_dims(B, H, Hk, D, dtype);
   if (rc) return rc;
   if ((rc = check_bf16_operand("q", q, sq_b, sq_h, sq_m, sq_d))) return rc;
@@ -411,7 +411,8 @@ int attn_fwd_common(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m, int
                                            kv_idx, si_b, si_h, si_t, B, H, Hk, M, N, D, dtype, Qt,
                                            k_slots, block_m, scale, static_cast<uint16_t*>(out),
                                            so_b, so_h, so_m, st, rowmask,
-                                           reinterpret_cast<int32_t*>(vt + kv_copy_elems(B, Hk, N, D))),
+                                           reinterpret_cast<int32_t*>(vt + kv_copy_elems(B, Hk, N, D)),
+                                           lists_grow),
                     "attn_fwd");
 }
 
@@ -446,6 +447,21 @@ int ugbsa_attn_fwd_rows(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m,
                          sv_n, sv_d, kv_idx, rowmask, si_b, si_h, si_t, si_s, B, H, Hk, M, N, D,
                          dtype, Qt, k_slots, block_m, scale, out, so_b, so_h, so_m, so_d,
                          workspace, workspace_elems, stream);
+}
+
+int ugbsa_attn_fwd_rows_grow(const void* q, int64_t sq_b, int64_t sq_h, int64_t sq_m, int64_t sq_d,
+                             const void* k, int64_t sk_b, int64_t sk_h, int64_t sk_n, int64_t sk_d,
+                             const void* v, int64_t sv_b, int64_t sv_h, int64_t sv_n, int64_t sv_d,
+                             const int32_t* kv_idx, const uint64_t* rowmask, int64_t si_b,
+                             int64_t si_h, int64_t si_t, int64_t si_s, int B, int H, int Hk, int M,
+                             int N, int D, int dtype, int Qt, int k_slots, int block_m, float scale,
+                             void* out, int64_t so_b, int64_t so_h, int64_t so_m, int64_t so_d,
+                             void* workspace, int64_t workspace_elems, void* stream) {
+  if (rowmask == nullptr) return fail(UGBSA_EARG, "rowmask is null");
+  return attn_fwd_common(q, sq_b, sq_h, sq_m, sq_d, k, sk_b, sk_h, sk_n, sk_d, v, sv_b, sv_h,
+                         sv_n, sv_d, kv_idx, rowmask, si_b, si_h, si_t, si_s, B, H, Hk, M, N, D,
+                         dtype, Qt, k_slots, block_m, scale, out, so_b, so_h, so_m, so_d,
+                         workspace, workspace_elems, stream, true);
 }
 
 int ugbsa_keep_kv_idx(const uint8_t* keep, int B, int H, int M, int NB, int block_m,

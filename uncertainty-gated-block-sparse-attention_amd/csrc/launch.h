@@ -117,7 +117,7 @@ hipError_t launch_attn_fwd(const uint16_t* q, int64_t sq_b, int64_t sq_h, int64_
                            int D, int elem, int Qt, int k_slots, int block_m, float scale,
                            uint16_t* out, int64_t so_b, int64_t so_h, int64_t so_m,
                            hipStream_t stream, const uint64_t* rowmask = nullptr,
-                           int32_t* order_ws = nullptr);
+                           int32_t* order_ws = nullptr, bool lists_grow = false);
 
 // LDS bytes of one wavefront of the 64-row-tile kernels.
 int attn_wave_lds(int N, int D, int k_slots, bool row_masks);

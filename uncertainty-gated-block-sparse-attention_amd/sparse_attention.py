@@ -313,6 +313,7 @@ def _select_logged(query, key_states, scaling, block_m=64, planes=None, mode=Non
 # together (under PROF the copies stay in the v2_kernel bucket, apart from the
 # selector's launches in v2_select).
 _AS_DEFINED = (_block_select_kv_idx_v2, select_v2, block_summary, block_sparse_attn_v2)
+_ROWS_AS_DEFINED = block_sparse_attn
 
 
 def _prepare_layer(query, key, value):
@@ -592,8 +593,10 @@ def block_sparse_attention(module, query, key, value, attention_mask,
     B, _, S, D = query.shape
     out = torch.empty(B, S, H, D, dtype=query.dtype, device=query.device)
     ws = attn_workspace(B, Hk, key.shape[-2], D, query.device)
+    # the selector's lists grow with the tile (a replaced launcher keeps its arguments)
+    hint = {"lists_grow": True} if block_sparse_attn is _ROWS_AS_DEFINED else {}
     block_sparse_attn(query, key, value, keep, scale=scaling, block_n=BLOCK,
-                      out=out.transpose(1, 2), workspace=ws)
+                      out=out.transpose(1, 2), workspace=ws, **hint)
     return out, None
 
 
