@@ -9,7 +9,7 @@ import dump_block_scores as dbs
 import sparse_attention as sa
 import synth
 from oracle import score_dump as OD
-from parity import f32np
+from parity import f32np, same_float_bits
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
@@ -28,13 +28,18 @@ def test_tau_splits(hip_lib, S, D, mode, score, dtype):
     q, k, _ = synth.make_layer(synth.CONFIGS["c1"], 3, S=S, Hq=4, Hkv=2, D=D, dtype=dtype)
     sel = sa.Selector()
     sel.mode, sel.router_score, sel.budget_blocks = mode, score, 1
-    shard = dbs.record(q.to(DEV), k.to(DEV), D ** -0.5, sel=sel)
+    shard = dbs.record(q.to(DEV), k.to(DEV), D ** -0.5, sel=sel, want_tile_score=True)
     ref = OD.tau_hat(f32np(q), f32np(k), D ** -0.5, sa.use_quest(sel))
     # fp32 scores of both: a difference of two rows' scores, of the scores' own size, carries
     # at most a few times D 2^-24 of it, and the mean of their squares less
     np.testing.assert_allclose(shard["tau_hat"], ref, rtol=1e-4)
-    for name in ("g", "r", "sigma", "g_rho"):       # no partial sum left in the arrays
-        assert (shard[name][..., shard["valid"]] <= 2 * np.abs(shard["r"]).max()).all()
+    # no partial sum left in g or r, the tiles past the valid ones among them: the order
+    # statistics of the kernel's own scores, bit for bit
+    T = shard["tile_score"].cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        stats = OD.order_stats(T, *OD.dump_budgets(sel.budget_blocks, T.shape[-1]))
+    for name, want in zip(("g", "r", "sigma", "g_rho"), stats):
+        assert same_float_bits(shard[name], want), name
     again = dbs.record(q.to(DEV), k.to(DEV), D ** -0.5, sel=sel)
     for name in ("g", "r", "sigma", "g_rho", "valid", "tau_hat"):
         assert np.array_equal(shard[name], again[name], equal_nan=True), name

@@ -34,7 +34,7 @@ constexpr int kTauWaves = 8;
 constexpr int kTauMaxPairs = 1024;   // n_pairs cap of the reference
 constexpr int kTauTarget = 512;      // workgroups that fill the chip
 
-// Blocks per LDS chunk: 16 KiB of planes.
+// Blocks per LDS chunk: 16 KiB of planes (8 at head_dim 64).
 __host__ __device__ constexpr int tau_chunk(int D) { return D > 128 ? 16 : 32; }
 
 template <typename E, int D, bool QUEST, int MT>
