@@ -906,7 +906,10 @@ static int resident_workgroups(Kern kern, int threads, size_t lds) {
 // 89 % of the re-reads) one launch, 2.13 against 2.30 / 2.23 / 2.20 / 2.19.
 // The fabric traffic of the c3 launch falls from 120 GB to about 20 GB.  A
 // fractional multiple leaves a partial last wave in every launch (x1.5:
-// 22.4 ms at c3).
+// 22.4 ms at c3).  Head_dim 64, whose resident wave is 2048 workgroups: 16 heads x
+// 64K, lists of up to 256, one launch 3.1-3.3 / 4.2 / 3.7 / 3.46 / 3.25; x 128K 7.65
+// / 8.85 / 8.26 / 8.07 / 7.94; 28 heads x 64K, lists of 96, 2.97 / 3.28 / 3.16 / 3.10
+// / 3.08 (with one wavefront per SIMD, generations of 3x 1024: 4.25, 8.70, 3.57).
 template <int D>
 constexpr int gen_waves() { return D > 128 ? 1 : 3; }
 
