@@ -23,12 +23,18 @@ def check(out, ref):
     assert err.max() <= MAX_ABS and err.mean() <= MEAN_ABS, (err.max(), err.mean())
 
 
-# (H, M): 12 tiles and 72 (four wavefronts a tile), 360 (two), 720 (one); lists from none to every
-# visible block, so runs of no, one and several blocks, and one list in slot order (repeats)
+# (H, M) with one, two and four wavefronts per tile at every head_dim that has them, for lists as
+# wide as the context and for row masks (test_layer_route_cpu.py asks the library which each takes)
+LISTS = [(4, 190), (4, 1150), (20, 1101), (40, 1150), (56, 1101)]
+ROWS = [(4, 190), (4, 1150), (28, 1101), (56, 1101)]
+
+
+# lists from none to every visible block, so runs of no, one and several blocks, and one list in
+# slot order (repeats)
 @pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float16),
                                      (128, torch.bfloat16), (128, torch.float16),
                                      (256, torch.bfloat16), (256, torch.float16)])
-@pytest.mark.parametrize("H,M", [(4, 190), (4, 1150), (20, 1101), (40, 1150)])
+@pytest.mark.parametrize("H,M", LISTS)
 def test_tile_lists(hip_lib, D, dtype, H, M):
     print(f"[case] split lists D={D} {dtype} H={H} M={M}", flush=True)
     q, k, v = qkv(H + M + D, 1, H, H // 2, M, D, dtype)
@@ -55,7 +61,7 @@ def test_tile_lists(hip_lib, D, dtype, H, M):
 
 
 @pytest.mark.parametrize("D", [64, 128, 256])
-@pytest.mark.parametrize("H,M", [(4, 190), (20, 1101)])
+@pytest.mark.parametrize("H,M", ROWS)
 def test_row_masks(hip_lib, D, H, M):
     print(f"[case] split row masks D={D} H={H} M={M}", flush=True)
     q, k, v = qkv(H + M + D, 1, H, H // 2, M, D, torch.bfloat16)

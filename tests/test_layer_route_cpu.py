@@ -166,3 +166,17 @@ def test_row_masked_calls_say_whether_their_lists_grow(rec, monkeypatch):
                         lambda q, k, v, keep, scale, block_n, out, workspace: seen.append(1))
     sa.block_sparse_attention(module, q, k, v, None, 0.125)
     assert seen == [1]
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_split_shapes_cover_every_form(D):
+    """The calls of test_gpu_attention_split.py launch every number of wavefronts per tile."""
+    import test_gpu_attention_split as split
+    lib = _capi.lib()
+
+    def forms(shapes, row_masks):
+        return {lib.ugbsa_attn_tile_waves(1, H, M, D, (M + 63) // 64, row_masks) for H, M in shapes}
+    assert forms(split.LISTS, 0) == {1, 2, 4}
+    assert forms(split.ROWS, 1) == ({1, 2, 4} if D < 256 else {1})     # no split row-masked form there
+    past = lib.ugbsa_attn_tile_waves(1, 1, 64 * 530 - 9, D, 40, 0)     # its long contexts
+    assert past == (4 if D == 64 else 1)

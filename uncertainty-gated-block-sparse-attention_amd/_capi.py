@@ -61,6 +61,7 @@ SIGNATURES = {
                                       _p, _p, _i64, _i64, _i64, _i64,
                                       _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _f,
                                       _p, _i64, _i64, _i64, _i64, _p, _i64, _p]),
+    "ugbsa_attn_tile_waves": (_i64, [_i, _i, _i, _i, _i, _i]),
     "ugbsa_attn_wave_lds": (_i64, [_i, _i, _i, _i]),
     "ugbsa_attn_workspace_elems": (_i64, [_i, _i, _i, _i]),
     "ugbsa_attn_prepare_kv": (_i, [_p, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64,

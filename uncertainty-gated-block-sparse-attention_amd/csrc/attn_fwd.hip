@@ -284,6 +284,11 @@ static int attn_split(int64_t tiles, int Qt, int k_slots, int NB, int D, bool ro
   return best;
 }
 
+int attn_tile_waves(int B, int H, int N, int D, int k_slots, bool row_masks) {
+  const int NB = (N + kBlock - 1) / kBlock;
+  return attn_split(static_cast<int64_t>(B) * H * NB, NB, k_slots, NB, D, row_masks);
+}
+
 hipError_t launch_attn_prepare(const uint16_t* k, int64_t sk_b, int64_t sk_h, int64_t sk_n,
                                const uint16_t* v, int64_t sv_b, int64_t sv_h, int64_t sv_n,
                                int B, int Hk, int N, int D, int block_m, uint16_t* ws,
@@ -569,7 +574,7 @@ static hipError_t launch_attn_fwd_e(const uint16_t* q, int64_t sq_b, int64_t sq_
     if (k_slots > kPipeMaxSlots) return hipErrorInvalidValue;
     const int NBk = (N + kBlock - 1) / kBlock;
     const int64_t tiles = static_cast<int64_t>(B) * H * Qt;
-    const int split = attn_split(tiles, Qt, k_slots, NBk, D, rowmask != nullptr);
+    const int split = attn_tile_waves(B, H, N, D, k_slots, rowmask != nullptr);   // M == N
     const int32_t* tile_order = nullptr;
     // Not ranked: calls whose wavefronts all start at once, and calls in one launch
     // whose caller knows that the lists grow with t, as the per-row selector's unions

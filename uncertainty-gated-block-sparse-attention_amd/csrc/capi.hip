@@ -475,6 +475,10 @@ int ugbsa_keep_kv_idx(const uint8_t* keep, int B, int H, int M, int NB, int bloc
                     "keep_kv_idx");
 }
 
+int64_t ugbsa_attn_tile_waves(int B, int H, int N, int D, int k_slots, int row_masks) {
+  return ugbsa::attn_tile_waves(B, H, N, D, k_slots, row_masks != 0);
+}
+
 int64_t ugbsa_attn_wave_lds(int N, int D, int k_slots, int row_masks) {
   return ugbsa::attn_wave_lds(N, D, k_slots, row_masks != 0);
 }

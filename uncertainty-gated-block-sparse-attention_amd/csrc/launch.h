@@ -119,7 +119,8 @@ hipError_t launch_attn_fwd(const uint16_t* q, int64_t sq_b, int64_t sq_h, int64_
                            hipStream_t stream, const uint64_t* rowmask = nullptr,
                            int32_t* order_ws = nullptr, bool lists_grow = false);
 
-// LDS bytes of one wavefront of the 64-row-tile kernels.
+// Wavefronts per 64-row tile of a call, and the LDS bytes of one of them.
+int attn_tile_waves(int B, int H, int N, int D, int k_slots, bool row_masks);
 int attn_wave_lds(int N, int D, int k_slots, bool row_masks);
 
 // The (b, t) tiles of a kv_idx [B, H, Qt, k_slots] ordered by their visited
