@@ -23,7 +23,7 @@
 //
 // 28 heads x 4096 rows x 64 blocks: 35 us (a radix select through LDS
 // histograms, a 64-bit sort and LDS flags took 119); 8 x 10007 x 157, belief:
-// 87 us (117).
+// 91 us (117).
 #include "common.h"
 #include "launch.h"
 
