@@ -223,11 +223,12 @@ int ugbsa_attn_fwd_rows_grow(const void* q, int64_t sq_b, int64_t sq_h, int64_t 
                              void* workspace, int64_t workspace_elems, void* stream);
 
 /* Wavefronts that share each 64-row tile's list in an attention call of these
- * sizes (k_slots slots a list; row_masks != 0: the rows entry points): 1, 2 or 4. */
+ * sizes (k_slots slots a list; row_masks != 0: the rows entry points): 1, 2 or 4,
+ * 0 for sizes that no call takes. */
 int64_t ugbsa_attn_tile_waves(int B, int H, int N, int D, int k_slots, int row_masks);
 
 /* LDS bytes that one wavefront of the 64-row-tile attention takes for Q, the
- * list of a tile of k_slots slots and (row_masks != 0) its masks. */
+ * list of a tile of k_slots slots and (row_masks != 0) its masks; 0 likewise. */
 int64_t ugbsa_attn_wave_lds(int N, int D, int k_slots, int row_masks);
 
 /* Number of 16-bit elements of the attention workspace, in two parts:

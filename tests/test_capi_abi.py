@@ -168,3 +168,12 @@ def test_decode_calls_without_a_workspace(lib):
     for B, H, Hk, D in ((1, 1, 1, 64), (1, 28, 4, 128), (3, 64, 1, 256), (64, 64, 64, 128)):
         assert all(lib.ugbsa_decode_workspace_elems(B, H, Hk, n, D) == 0 for n in range(1, line))
     assert lib.ugbsa_decode_workspace_elems(1, 28, 4, line, 128) > 0
+
+
+def test_form_queries_of_sizes_no_call_takes(lib):
+    for B, H, N, D, k in ((0, 4, 64, 128, 1), (1, 0, 64, 128, 1), (1, 4, 0, 128, 1), (1, 4, 64, 96, 1),
+                          (1, 4, 64, 128, 0), (1, 4, 64, 128, -2)):
+        assert lib.ugbsa_attn_tile_waves(B, H, N, D, k, 0) == 0
+    assert lib.ugbsa_attn_wave_lds(0, 128, 1, 1) == lib.ugbsa_attn_wave_lds(64, 96, 1, 1) == 0
+    assert lib.ugbsa_attn_wave_lds(64, 128, -2, 0) == 0
+    assert lib.ugbsa_attn_tile_waves(1, 4, 64, 128, 1, 0) == 1 and lib.ugbsa_attn_wave_lds(64, 128, 1, 0) > 0

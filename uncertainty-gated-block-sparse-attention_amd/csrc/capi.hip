@@ -476,10 +476,12 @@ int ugbsa_keep_kv_idx(const uint8_t* keep, int B, int H, int M, int NB, int bloc
 }
 
 int64_t ugbsa_attn_tile_waves(int B, int H, int N, int D, int k_slots, int row_masks) {
+  if (check_dims(B, H, 1, D, UGBSA_DTYPE_BF16) || N < 1 || k_slots < 1) return 0;
   return ugbsa::attn_tile_waves(B, H, N, D, k_slots, row_masks != 0);
 }
 
 int64_t ugbsa_attn_wave_lds(int N, int D, int k_slots, int row_masks) {
+  if (check_dims(1, 1, 1, D, UGBSA_DTYPE_BF16) || N < 1 || k_slots < 1) return 0;
   return ugbsa::attn_wave_lds(N, D, k_slots, row_masks != 0);
 }
 
