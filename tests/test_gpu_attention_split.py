@@ -173,3 +173,21 @@ def test_tile_order_of_row_masks(hip_lib, D):
     assert torch.equal(ranked, block_sparse_attn(q, k, v, keep, D ** -0.5, lists_grow=True))
     check(ranked[:, :1], OA.keep_attention(f32np(q[:, :1]), f32np(k[:, :1]), f32np(v[:, :1]),
                                            keep[:, :1].cpu().numpy(), D ** -0.5))
+
+
+def test_row_masks_in_a_graph(hip_lib):
+    """A context whose lists are worth asking the device for their longest is captured without."""
+    M, D = 64 * 700, 256
+    q, k, v = (t.to(DEV) for t in qkv(9, 1, 2, 1, M, D, torch.bfloat16))
+    tile, nbs = torch.arange(M, device=DEV) // 64, torch.arange(700, device=DEV)
+    keep = ((tile[:, None] == nbs) | (nbs == 0)).expand(1, 2, M, 700).contiguous()
+    eager = block_sparse_attn(q, k, v, keep, D ** -0.5)
+    out, graph = torch.empty_like(q), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        block_sparse_attn(q, k, v, keep, D ** -0.5, out=out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        assert torch.equal(block_sparse_attn(q, k, v, keep, D ** -0.5), eager)

@@ -48,6 +48,7 @@ def rec(monkeypatch):
     rec = Recorder(_capi.lib())
     monkeypatch.setattr(_capi, "lib", lambda: rec)
     monkeypatch.setattr(_capi, "stream_ptr", lambda device: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     monkeypatch.setattr(sa, "SEL", sa.Selector())
     sa.SEL.mode, sa.SEL.kernel_v2, sa.SEL.budget_blocks = "router", True, 8
     sa.SEL.k_min = 2

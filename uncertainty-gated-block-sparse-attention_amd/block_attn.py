@@ -208,8 +208,10 @@ _CU_LDS = 160 * 1024
 
 
 def _list_as_wide_as_mask(N, D, NB, block_m):
-    return (block_m == 64 and NB <= _ROWS_LIST_BLOCKS
-            and (8 if D == 64 else 4) * _capi.lib().ugbsa_attn_wave_lds(N, D, NB, 1) <= _CU_LDS)
+    if block_m != 64 or NB > _ROWS_LIST_BLOCKS:
+        return False
+    return ((8 if D == 64 else 4) * _capi.lib().ugbsa_attn_wave_lds(N, D, NB, 1) <= _CU_LDS
+            or torch.cuda.is_current_stream_capturing())      # no question to the device there
 
 
 def block_sparse_attn(q, k, v, keep, scale, block_n=64, block_m=64,
